@@ -10,12 +10,9 @@
 // One pass = two kernels over the current worklist W (cell ids):
 //   k_sweep  evaluates, for every listed cell at its current alpha, e_q = exp(alpha.m_q),
 //            sum_q w_q e_q and H = M^T diag(w e) M.  A wavefront takes 4 cells; the block's
-//            16 cells share every M chunk staged in LDS, each lane computes one ordinate's
-//            exponent for the 4 cells (fused multiply-adds in moment order), and the four
-//            Hessians accumulate on the matrix cores (V_MFMA_F64_16X16X4_F64, 4 ordinates
-//            per instruction, A = (w e m_q)^T, B = m_q; nm = 25 uses the three 16x16 tiles
-//            of the lower block triangle).  Operand lanes: A[i][k], B[k][j] sit in lane
-//            16k + i (16k + j); accumulator register r of lane l holds D[l/16 + 4r][l%16].
+//            16 cells share every M chunk staged in LDS, and the four cells' lower-triangle
+//            4x4 blocks of H accumulate on the matrix cores (V_MFMA_F64_4X4X4_4B_F64, one
+//            cell per block slot: Quad).  H is stored as its packed lower triangle.
 //   k_step   advances each listed cell by exactly one step of its state machine with that
 //            sweep's result: either the Armijo test of a line-search trial, or one Newton
 //            iteration (Cholesky in dpotf2 order, the dlacn2/dtrsv condition estimate, the
@@ -864,13 +861,18 @@ struct MixedChunk {
     }
 };
 
+// LDS row stride of the quad sweep's M chunks: even, so that a row starts on 16 bytes, and
+// 2 mod 4 doubles, so that 16 consecutive rows start in 16 distinct groups of four banks (the
+// exponent chains read 16 rows at a time as pairs of doubles, without conflicts).
+__host__ __device__ constexpr int quad_stride(int nm) { return nm % 2 ? nm + 1 : nm + 2; }
+
 // M and w chunks of kChunk ordinates staged through double-buffered LDS by a whole block:
 // each thread holds its share of the next chunk in registers while the block consumes the
 // current one, so one barrier per chunk publishes a chunk and the global loads overlap the
 // matrix-core work.
 template <int NM>
 struct ChunkStager {
-    static constexpr int NMS = NM | 1;
+    static constexpr int RS = quad_stride(NM);
     static constexpr int kPer = (kChunk * NM + kBlock - 1) / kBlock;
     double pre[kPer];
     double prew;
@@ -892,7 +894,7 @@ struct ChunkStager {
             const int e = tid + kBlock * k;
             if (e < kChunk * NM) {
                 const int rr = e / NM, cc = e - rr * NM;
-                sM[rr * NMS + cc] = pre[k];
+                sM[rr * RS + cc] = pre[k];
             }
         }
         if (tid < kChunk)
@@ -900,128 +902,175 @@ struct ChunkStager {
     }
 };
 
-// The chunk ordinate whose exponent and weight lane l computes in the FP64 sweep.
+// Row i of the packed lower triangle starts at i (i + 1) / 2.
+__host__ __device__ constexpr int tri(int i) { return i * (i + 1) / 2; }
+
+// The chunk ordinate whose exponent and weight lane l computes in the tail's FP64 sweep.
 __device__ __forceinline__ int mfma_ordinate(int lane) { return lane; }
 
-// Matrix-core accumulation of one LDS chunk of kChunk ordinates for CW cells: lane l owns
-// ordinate mfma_ordinate(l) of the chunk for the exponent (wl is that ordinate's weight),
-// then the MFMA loop consumes 4 ordinates per instruction.  The operation sequence per cell
-// does not depend on CW or on the other cells of the wave, so a cell's H is the same bits
+// Matrix-core accumulation of one LDS chunk of kChunk ordinates for one cell (the tail's lone
+// cells): lane l owns ordinate mfma_ordinate(l) of the chunk for the exponent (wl is that
+// ordinate's weight), then the MFMA loop consumes 4 ordinates per instruction.  The operation
+// sequence per element of H and of f is chunk_quad's, so a cell's sweep is the same bits
 // whichever kernel evaluates it.
-template <int NM, int CW>
+template <int NM>
 __device__ __forceinline__ void chunk_mfma(const double *sMc, double wl, const double *sAc,
-                                           d4 (&acc)[CW][(NM + 15) / 16 * ((NM + 15) / 16 + 1) / 2],
-                                           double (&fpart)[CW], int lane)
+                                           d4 (&acc)[(NM + 15) / 16 * ((NM + 15) / 16 + 1) / 2],
+                                           double &fpart, int lane)
 {
     constexpr int NT = (NM + 15) / 16;
     constexpr int NMS = NM | 1;
     const int gq = lane >> 4, rq = lane & 15;
     const double *rowp = &sMc[mfma_ordinate(lane) * NMS];
-    double we[CW];
+    double x = 0.0;
 #pragma unroll
-    for (int c = 0; c < CW; ++c) {
-        double x = 0.0;
-#pragma unroll
-        for (int i = 0; i < NM; ++i)
-            x = fma(sAc[c * NM + i], rowp[i], x);
-        we[c] = wl * exp(x);
-        fpart[c] = fpart[c] + we[c];
-    }
+    for (int i = 0; i < NM; ++i)
+        x = fma(sAc[i], rowp[i], x);
+    const double we = wl * exp(x);
+    fpart = fpart + we;
 #pragma unroll
     for (int k = 0; k < kChunk / 4; ++k) {
         const int ql = 4 * k + gq;
         const double *mr = &sMc[ql * NMS];
         const double b0 = (rq < NM) ? mr[rq] : 0.0;
         const double b1 = (NT == 2 && 16 + rq < NM) ? mr[16 + rq] : 0.0;
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            const double wq = __shfl(we[c], ql);
-            acc[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b0, b0, acc[c][0], 0, 0, 0);
-            if constexpr (NT == 2) {
-                acc[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b0, acc[c][1], 0, 0, 0);
-                acc[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b1, acc[c][2], 0, 0, 0);
-            }
+        const double wq = __shfl(we, ql);
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b0, b0, acc[0], 0, 0, 0);
+        if constexpr (NT == 2) {
+            acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b0, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b1, acc[2], 0, 0, 0);
         }
     }
 }
 
-// chunk_mfma for four cells and nm <= 9 on V_MFMA_F64_4X4X4_4B_F64 (as fast per flop as the
-// 16x16 instruction): the lower-triangle 4x4 blocks (R, C) of H, one instruction per block
-// with the four cells in its four block slots, in place of a 16x16 tile per cell of which
-// nm^2 entries are used.  Lane l: cell (l >> 2) & 3, row or column l & 3 of the block, K index
-// l >> 4 (ordinate 4 k + (l >> 4) of K step k, as in chunk_mfma).  Each element's chain of
-// fused multiply-adds over the ordinates, and its operands w_q m_qi (rounded) and m_qj, are
-// chunk_mfma's, so H has the same bits; the exponents and f are chunk_mfma's code.
+// Lane C of the lane's quad (four consecutive lanes), on the vector unit.
+template <int C>
+__device__ __forceinline__ double quad_bcast(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), C * 0x55, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), C * 0x55, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// The bulk FP64 sweep of four cells a wave on V_MFMA_F64_4X4X4_4B_F64 (as fast per flop as the
+// 16x16 instruction): H's lower-triangle 4x4 blocks (R, C), one instruction per block and four
+// ordinates with the four cells in its four block slots.  Against a 16x16 tile per cell that is
+// 6 blocks' work instead of 16 at nm = 9, 10 of 16 at nm = 16 and 28 of 48 at nm = 25.
+//
+// Lane l: cell (l >> 2) & 3, row or column l & 3 of the block, K index l >> 4 (ordinate
+// 4 k + (l >> 4) of K step k).  The exponents are laid out to match: the lane evaluates, for
+// its own cell (alpha in registers), the ordinates 4 k + (l >> 4) of the K steps k = 4 j +
+// (l & 3), j = 0..3, so a K step's weight sits in the lane's own quad and one quad broadcast on
+// the vector unit fetches it -- no LDS permutes, and the four cells share each M row they read.
+//
+// What bounds it: the FP64 matrix instructions (16 cycles each) and the FP64 vector work of the
+// exponents take turns on the SIMD; per chunk and wave 16 NBLK of the former and 4 (nm + ~40)
+// vector instructions of 4 cycles.  Measured against a 16x16 tile per cell with LDS-permuted
+// weights: H of 32771 M_3 cells at 1152 ordinates 281 us (449 before); the M_3 FP64 closure of
+// 150001 cells 30.3 ms (36.8); an M_2 step of 128^3 cells, whose earlier 4x4-block sweep
+// fetched its weights by LDS permutes, 64.8 ms (77.3).
 template <int NM>
-struct Blk4 {
+struct Quad {
     static constexpr int NR = (NM + 3) / 4;
     static constexpr int NBLK = NR * (NR + 1) / 2;
-};
-template <int NM>
-__device__ __forceinline__ void chunk_mfma4(const double *sMc, double wl, const double *sAc,
-                                            double (&acc)[Blk4<NM>::NBLK], double (&fpart)[4],
-                                            int lane)
-{
-    static_assert(NM <= 9, "the 16x16 tile serves larger orders");
-    constexpr int NR = Blk4<NM>::NR;
-    constexpr int NMS = NM | 1;
-    const double *rowp = &sMc[mfma_ordinate(lane) * NMS];
-    double we[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        double x = 0.0;
+    static constexpr int RS = quad_stride(NM);
+    // doubles of one chunk's rows: the last row's operand reads run to column 4 NR - 1
+    static constexpr int kRows = kChunk * RS + 4;
+
+    double al[NM];  // alpha of the lane's cell
+    double acc[NBLK];
+    double fp[4];  // sum of the weights of the lane's four ordinate slots
+
+    __device__ __forceinline__ void start(const double *alpha)
+    {
 #pragma unroll
         for (int i = 0; i < NM; ++i)
-            x = fma(sAc[c * NM + i], rowp[i], x);
-        we[c] = wl * exp(x);
-        fpart[c] = fpart[c] + we[c];
+            al[i] = alpha ? alpha[i] : 0.0;
+#pragma unroll
+        for (int p = 0; p < NBLK; ++p)
+            acc[p] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            fp[j] = 0.0;
     }
-    const int ii = lane & 3, kq = lane >> 4, cb = (lane >> 2) & 3;
+
+    template <int J>
+    __device__ __forceinline__ void ksteps(const double *sMc, double we, int lane)
+    {
+        const int ii = lane & 3, kq = lane >> 4;
+        auto step = [&](double wq, int k) {
+            // columns >= nm hold the next row's entries (finite); their outputs are not stored
+            const double *mr = &sMc[(4 * k + kq) * RS + ii];
+            double mv[NR];
 #pragma unroll
-    for (int k = 0; k < kChunk / 4; ++k) {
-        const int ql = 4 * k + kq;
-        const double *mr = &sMc[ql * NMS];
-        double mv[NR];
+            for (int r = 0; r < NR; ++r)
+                mv[r] = mr[4 * r];
+            int p = 0;
 #pragma unroll
-        for (int r = 0; r < NR; ++r)
-            mv[r] = (4 * r + ii < NM) ? mr[4 * r + ii] : 0.0;
-        double w4[4];
+            for (int R = 0; R < NR; ++R) {
+                const double a = wq * mv[R];
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            w4[c] = __shfl(we[c], ql);
-        const double wq = cb == 0 ? w4[0] : (cb == 1 ? w4[1] : (cb == 2 ? w4[2] : w4[3]));
+                for (int C = 0; C <= R; ++C) {
+                    acc[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, mv[C], acc[p], 0, 0, 0);
+                    ++p;
+                }
+            }
+        };
+        step(quad_bcast<0>(we), 4 * J);
+        step(quad_bcast<1>(we), 4 * J + 1);
+        step(quad_bcast<2>(we), 4 * J + 2);
+        step(quad_bcast<3>(we), 4 * J + 3);
+    }
+
+    __device__ __forceinline__ void chunk(const double *sMc, const double *sWc, int lane)
+    {
+        const int o = 4 * (lane & 3) + (lane >> 4);  // the lane's ordinate slot at j = 0
+        double we[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const double *rowp = &sMc[(16 * j + o) * RS];
+            double x = 0.0;
+#pragma unroll
+            for (int i = 0; i < NM; ++i)
+                x = fma(al[i], rowp[i], x);
+            we[j] = sWc[16 * j + o] * exp(x);
+            fp[j] = fp[j] + we[j];
+        }
+        ksteps<0>(sMc, we[0], lane);
+        ksteps<1>(sMc, we[1], lane);
+        ksteps<2>(sMc, we[2], lane);
+        ksteps<3>(sMc, we[3], lane);
+    }
+
+    // sum_q w_q e_q of the lane's cell (every lane of the cell): wave_sum's butterfly over the
+    // ordinate slots 16 j + 4 (l & 3) + (l >> 4), bit 5 of the slot first
+    __device__ __forceinline__ double f() const
+    {
+        double s = (fp[0] + fp[2]) + (fp[1] + fp[3]);
+        s = s + __shfl_xor(s, 2);
+        s = s + __shfl_xor(s, 1);
+        s = s + __shfl_xor(s, 32);
+        s = s + __shfl_xor(s, 16);
+        return s;
+    }
+
+    // put(i, j, value) for the lane's elements of its cell's lower triangle
+    template <typename F>
+    __device__ __forceinline__ void each(F put, int lane) const
+    {
+        const int i0 = lane >> 4, j0 = lane & 3;
         int p = 0;
 #pragma unroll
-        for (int R = 0; R < NR; ++R) {
-            const double a = wq * mv[R];
+        for (int R = 0; R < NR; ++R)
 #pragma unroll
             for (int C = 0; C <= R; ++C) {
-                acc[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, mv[C], acc[p], 0, 0, 0);
+                const int i = 4 * R + i0, j = 4 * C + j0;
+                if (i < NM && j <= i)
+                    put(i, j, acc[p]);
                 ++p;
             }
-        }
     }
-}
-
-// H of the lane's cell from chunk_mfma4's blocks: element (4 R + (l >> 4), 4 C + (l & 3)),
-// lower triangle, mirrored (store_H's writes).
-template <int NM>
-__device__ __forceinline__ void store_H4(const double (&acc)[Blk4<NM>::NBLK], double *H, int lane)
-{
-    const int i0 = lane >> 4, j0 = lane & 3;
-    int p = 0;
-#pragma unroll
-    for (int R = 0; R < Blk4<NM>::NR; ++R)
-#pragma unroll
-        for (int C = 0; C <= R; ++C) {
-            const int i = 4 * R + i0, j = 4 * C + j0;
-            if (i < NM && j < NM && j <= i) {
-                H[i * NM + j] = acc[p];
-                H[j * NM + i] = acc[p];
-            }
-            ++p;
-        }
-}
+};
 
 // H from one cell's accumulators: lower triangle, mirrored (fobj.cpp:96-101).
 template <int NM>
@@ -1191,56 +1240,31 @@ __device__ __forceinline__ void store_H_ref(const RefEntries<NM> &E,
 }
 
 // ---------------------------------------------------------------- sweep pass
-// A wavefront takes 4 cells; the block's 16 cells share every M chunk staged in LDS.
+// A wavefront takes 4 cells (Quad); the block's 16 cells share every M chunk staged in LDS.
+// Writes H as its packed lower triangle, which is all the step pass reads.
 template <int NM>
 __global__ __launch_bounds__(kBlock) void k_sweep(KParams P, const double *__restrict__ Mg,
                                                    const double *__restrict__ wg, State S,
                                                    const int *__restrict__ W,
                                                    const int *__restrict__ nWp)
 {
-    constexpr int NT = (NM + 15) / 16;
-    constexpr int NB = NT * (NT + 1) / 2;
-    constexpr int NMS = NM | 1;
     constexpr int CW = kCellsPerWave;
-    __shared__ double sM[2][kChunk * NMS];
+    __shared__ __align__(16) double sM[2][Quad<NM>::kRows];
     __shared__ double sW[2][kChunk];
-    __shared__ double sA[kWavesPerBlock][CW * NM];
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int nch = P.nqPad / kChunk;
     const int nW = uniform_int(*nWp);
     const int groups = (nW + CW - 1) / CW;
     const int nBlocksNeeded = (groups + kWavesPerBlock - 1) / kWavesPerBlock;
+    for (int e = tid; e < 2 * Quad<NM>::kRows; e += kBlock)
+        (&sM[0][0])[e] = 0.0;  // the pad columns are read as (unused) operands
     for (int blk = blockIdx.x; blk < nBlocksNeeded; blk += gridDim.x) {
         const int grp = blk * kWavesPerBlock + wv;
-        int cells[CW];
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            const int slot = grp * CW + c;
-            cells[c] = (grp < groups && slot < nW) ? W[slot] : -1;
-        }
-#pragma unroll
-        for (int c = 0; c < CW; ++c)
-            if (lane < NM)
-                sA[wv][c * NM + lane] =
-                    cells[c] >= 0 ? S.vec[(size_t)cells[c] * kVec * NM + kVa * NM + lane] : 0.0;
-        constexpr bool B4 = NM <= 9;  // 4x4 blocks, the four cells in the block slots
-        static_assert(!B4 || CW == 4, "one cell per block slot");
-        d4 acc[B4 ? 1 : CW][B4 ? 1 : NB];
-        double acc4[Blk4<B4 ? NM : 4>::NBLK];
-#pragma unroll
-        for (int c = 0; c < (B4 ? 1 : CW); ++c)
-#pragma unroll
-            for (int b = 0; b < (B4 ? 1 : NB); ++b)
-                acc[c][b] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int p = 0; p < Blk4<B4 ? NM : 4>::NBLK; ++p)
-            acc4[p] = 0.0;
-        double fpart[CW];
-#pragma unroll
-        for (int c = 0; c < CW; ++c)
-            fpart[c] = 0.0;
-        const bool any = cells[0] >= 0;
+        const int slot = grp * CW + ((lane >> 2) & 3);
+        const int cell = slot < nW ? W[slot] : -1;  // the lane's cell
+        Quad<NM> Q;
+        Q.start(cell >= 0 ? S.vec + (size_t)cell * kVec * NM + kVa * NM : nullptr);
         ChunkStager<NM> st;
         st.fetch(Mg, wg, 0, tid);
         __syncthreads();  // the previous cells' last chunk is consumed
@@ -1250,28 +1274,15 @@ __global__ __launch_bounds__(kBlock) void k_sweep(KParams P, const double *__res
             __syncthreads();
             if (ch + 1 < nch)
                 st.fetch(Mg, wg, ch + 1, tid);
-            if (any) {
-                if constexpr (B4)
-                    chunk_mfma4<NM>(sM[b], sW[b][mfma_ordinate(lane)], sA[wv], acc4, fpart, lane);
-                else
-                    chunk_mfma<NM, CW>(sM[b], sW[b][mfma_ordinate(lane)], sA[wv], acc, fpart,
-                                       lane);
-            }
+            if (grp < groups)
+                Q.chunk(sM[b], sW[b], lane);
         }
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            const double fs = wave_sum(fpart[c]);
-            if (cells[c] < 0)
-                continue;
-            if (lane == 0)
-                S.fdir[cells[c]] = fs;
-            if constexpr (!B4)
-                store_H<NM>(acc[c], S.H + (size_t)cells[c] * NM * NM, lane);
-        }
-        if constexpr (B4) {
-            const int cb = (lane >> 2) & 3;
-            if (cells[cb] >= 0)
-                store_H4<NM>(acc4, S.H + (size_t)cells[cb] * NM * NM, lane);
+        const double f = Q.f();
+        if (cell >= 0) {
+            if ((lane & 0x33) == 0)
+                S.fdir[cell] = f;
+            double *H = S.H + (size_t)cell * NM * NM;
+            Q.each([&](int i, int j, double v) { H[tri(i) + j] = v; }, lane);
         }
     }
 }
@@ -1441,9 +1452,6 @@ __device__ __forceinline__ void exp_arg4(const ExpA<NM> &A, BF b, double (&x)[4]
         for (int g = 0; g < 4; ++g)
             x[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(A.a[s], b(g, s), x[g], 0, 0, 0);
 }
-
-// Row i of the packed lower triangle starts at i (i + 1) / 2.
-__host__ __device__ constexpr int tri(int i) { return i * (i + 1) / 2; }
 
 // ---------------------------------------------------------------- column sweep (nm <= 25)
 // The mixed sweep for nm <= kPairMaxNm with the cells as the columns of its matrix products,
@@ -2178,8 +2186,9 @@ struct Cell {
     // in LDS or global memory; fdir = sum_q w_q e_q): either the Armijo test of a line-search
     // trial, or one Newton iteration of solveTheRest / optScaled.  sT: NM x (NM+1) doubles of
     // LDS for the transposed factor.  Returns 0 to continue, 1 converged, 2 ladder exhausted.
-    // H is not read when a line-search trial is rejected (it may then be null).
-    template <bool EXACT>
+    // H is not read when a line-search trial is rejected (it may then be null).  PACKED: H is
+    // the packed lower triangle in the FP64 phase too (the bulk sweeps' form).
+    template <bool EXACT, bool PACKED = false>
     __device__ __forceinline__ int advance(const KParams &P, const double *H, double fdir,
                                            const double *gm, double *sT, int lane)
     {
@@ -2209,10 +2218,12 @@ struct Cell {
         // ================================ one Newton iteration (solveTheRest)
         const bool mx = mixed(P);
         Dense<NM, EXACT, G> D;
-        if (mx) {  // the mixed sweep's packed lower triangle (all the mixed phase reads)
+        if (PACKED || mx) {  // the row's part above the diagonal mirrored (the mixed phase
+                             // does not read it)
 #pragma unroll
             for (int j = 0; j < NM; ++j)
-                D.row[j] = (own && j <= lane) ? H[tri(lane) + j] : 0.0;
+                D.row[j] = own && (j <= lane || !mx) ? H[j <= lane ? tri(lane) + j : tri(j) + lane]
+                                                     : 0.0;
         } else {
 #pragma unroll
             for (int j = 0; j < NM; ++j)
@@ -2415,7 +2426,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             Cell<NM, G> C;
             C.load(S, c, lane);
             const int done =
-                C.template advance<EXACT>(P, S.H + (size_t)c * NM * NM, S.fdir[c],
+                C.template advance<EXACT, !EXACT>(P, S.H + (size_t)c * NM * NM, S.fdir[c],
                                           S.vec + (size_t)c * kVec * NM + kVg * NM, sT[grp], lane);
             if (done) {
                 C.finish(done, c, u_g, alpha_g, stats, status, lane);
@@ -2805,11 +2816,11 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                     store_H_ref<NM>(E, h, sH, lane);
                     fdir = f;
                 } else {
-                    d4 acc[1][NB];
+                    d4 acc[NB];
 #pragma unroll
                     for (int b = 0; b < NB; ++b)
-                        acc[0][b] = d4{0.0, 0.0, 0.0, 0.0};
-                    double fpart[1] = {0.0};
+                        acc[b] = d4{0.0, 0.0, 0.0, 0.0};
+                    double fpart = 0.0;
                     double pre[NM];
                     const int qo = mfma_ordinate(lane);  // the lane's weight
                     double prew = wg[qo];
@@ -2833,11 +2844,11 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                             for (int k = 0; k < NM; ++k)
                                 pre[k] = Mg[base * NM + lane + kWave * k];
                         }
-                        chunk_mfma<NM, 1>(sM, wl, sA[0], acc, fpart, lane);
+                        chunk_mfma<NM>(sM, wl, sA[0], acc, fpart, lane);
                     }
                     wave_lds_sync();
-                    fdir = wave_sum(fpart[0]);
-                    store_H<NM>(acc[0], sH, lane);
+                    fdir = wave_sum(fpart);
+                    store_H<NM>(acc, sH, lane);
                 }
                 if (lane == 0)
                     sF[0] = fdir;
@@ -3115,7 +3126,8 @@ __global__ void k_budget(Lists L, c3d_cell_stats *stats, int *status)
     }
 }
 
-// H only (solveH_cuda / solveHMn semantics): one wave per cell.
+// H only (solveH_cuda / solveHMn semantics), row-major with both triangles: the bulk sweep's
+// four cells a wave.
 template <int NM>
 __global__ __launch_bounds__(kBlock) void k_hessian_fp64(int64_t ncells, int nqPad,
                                                         const double *__restrict__ Mg,
@@ -3123,67 +3135,37 @@ __global__ __launch_bounds__(kBlock) void k_hessian_fp64(int64_t ncells, int nqP
                                                         const double *__restrict__ alpha_g,
                                                         double *hs)
 {
-    constexpr int NT = (NM + 15) / 16;
-    constexpr int NB = NT * (NT + 1) / 2;
-    constexpr int NMS = NM | 1;
-    __shared__ double sM[kChunk * NMS];
-    __shared__ double sW[kChunk];
+    __shared__ __align__(16) double sM[2][Quad<NM>::kRows];
+    __shared__ double sW[2][kChunk];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int64_t cell = (int64_t)blockIdx.x * kWavesPerBlock + wv;
+    const int nch = nqPad / kChunk;
+    const int64_t cell = ((int64_t)blockIdx.x * kWavesPerBlock + wv) * kCellsPerWave +
+                         ((lane >> 2) & 3);
     const bool have = cell < ncells;
-    double as[NM];
-#pragma unroll
-    for (int i = 0; i < NM; ++i)
-        as[i] = have ? alpha_g[cell * NM + i] : 0.0;
-    d4 acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        acc[b] = d4{0.0, 0.0, 0.0, 0.0};
-    const int gq = lane >> 4, rq = lane & 15;
-    for (int c = 0; c < nqPad / kChunk; ++c) {
+    for (int e = tid; e < 2 * Quad<NM>::kRows; e += kBlock)
+        (&sM[0][0])[e] = 0.0;  // the pad columns are read as (unused) operands
+    Quad<NM> Q;
+    Q.start(have ? alpha_g + cell * NM : nullptr);
+    ChunkStager<NM> st;
+    st.fetch(Mg, wg, 0, tid);
+    __syncthreads();
+    for (int ch = 0; ch < nch; ++ch) {
+        const int b = ch & 1;
+        st.put(sM[b], sW[b], tid);
         __syncthreads();
-        for (int e = tid; e < kChunk * NM; e += kBlock) {
-            int rr = e / NM, cc = e - rr * NM;
-            sM[rr * NMS + cc] = Mg[(size_t)c * kChunk * NM + e];
-        }
-        if (tid < kChunk)
-            sW[tid] = wg[(size_t)c * kChunk + tid];
-        __syncthreads();
-        if (have) {
-            double x = 0.0;
-#pragma unroll
-            for (int i = 0; i < NM; ++i)
-                x = x + as[i] * sM[lane * NMS + i];
-            const double we = sW[lane] * exp(x);
-#pragma unroll
-            for (int k = 0; k < kChunk / 4; ++k) {
-                const int ql = 4 * k + gq;
-                const double wq = __shfl(we, ql);
-                const double b0 = (rq < NM) ? sM[ql * NMS + rq] : 0.0;
-                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b0, b0, acc[0], 0, 0, 0);
-                if constexpr (NT == 2) {
-                    const double b1 = (16 + rq < NM) ? sM[ql * NMS + 16 + rq] : 0.0;
-                    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b0, acc[1], 0, 0, 0);
-                    acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b1, acc[2], 0, 0, 0);
-                }
-            }
-        }
+        if (ch + 1 < nch)
+            st.fetch(Mg, wg, ch + 1, tid);
+        Q.chunk(sM[b], sW[b], lane);
     }
     if (!have)
         return;
     double *H = hs + cell * NM * NM;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int R = (b == 0) ? 0 : 1, Cb = (b == 2) ? 1 : 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int i = 16 * R + gq + 4 * k, j = 16 * Cb + rq;
-            if (i < NM && j < NM && j <= i) {
-                H[i * NM + j] = acc[b][k];
-                H[j * NM + i] = acc[b][k];
-            }
-        }
-    }
+    Q.each(
+        [&](int i, int j, double v) {
+            H[i * NM + j] = v;
+            H[j * NM + i] = v;
+        },
+        lane);
 }
 
 // H only, mixed mode, nm <= kPairMaxNm: the column sweep's Hessian under the cell's own shift
@@ -3658,7 +3640,8 @@ hipError_t launch_hessian_fp64(c3d_ctx_s *ctx, int64_t ncells, const double *alp
 {
     if (ncells <= 0)
         return hipSuccess;
-    dim3 grid((unsigned)((ncells + kWavesPerBlock - 1) / kWavesPerBlock));
+    constexpr int kCells = kWavesPerBlock * kCellsPerWave;
+    dim3 grid((unsigned)((ncells + kCells - 1) / kCells));
     if (ctx->precision == C3D_PREC_MIXED) {
 #define C3D_HC(NMV) hipLaunchKernelGGL(k_hessian_cols<NMV>, dim3((unsigned)ncells), dim3(kWave), 0, s, ncells, ctx->nqPad, ctx->d_M, ctx->d_wpad, (const _Float16 *)ctx->d_P16, ctx->d_R, alpha, hs)
         switch (ctx->t.nm) {
