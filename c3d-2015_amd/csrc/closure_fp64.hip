@@ -53,7 +53,7 @@ struct State {
     double *vec;   // [ncells][kVec][nm]
     double *scal;  // [ncells][kScal]
     int *ints;     // [ncells][kInt]
-    double *H;     // [ncells][nm][nm]
+    double *H;     // [ncells] of HBlock's doubles, in the reference order of nm * nm
     double *fdir;  // [ncells]  sum_q w_q e_q
 };
 
@@ -179,10 +179,10 @@ __device__ __forceinline__ float row16_max(float v)
     return v;
 }
 
-// A cell's lanes: the whole wave (G = 64, one cell per wave; broadcasts by readlane) or one
-// 16-lane row (G = 16, four cells per wave; broadcasts by DPP row_newbcast).  Lane indices
-// passed to the algebra below are indices within the group.  The arithmetic a cell sees is
-// the same in both layouts.
+// A cell's lanes: the whole wave (G = 64, one cell per wave; broadcasts by readlane), one
+// 16-lane row (G = 16, four cells per wave; broadcasts by DPP row_newbcast) or a quad (G = 4,
+// 16 cells per wave; broadcasts by DPP quad_perm).  Lane indices passed to the algebra below
+// are indices within the group.  The arithmetic a cell sees is the same in every layout.
 template <int G>
 struct Grp;
 
@@ -231,12 +231,55 @@ struct Grp<16> {
     {
         return __shfl(v, (int)(__lane_id() & 48u) + j);
     }
+    static __device__ __forceinline__ int first(int v)
+    {
+        return __builtin_amdgcn_mov_dpp(v, 0x150, 0xf, 0xf, false);
+    }
     static __device__ __forceinline__ bool all(bool p)
     {
         const unsigned long long b = __ballot(p);
         return ((b >> (__lane_id() & 48u)) & 0xFFFFull) == 0xFFFFull;
     }
 };
+
+// Lane C of the lane's quad (four consecutive lanes), on the vector unit.
+template <int C>
+__device__ __forceinline__ double quad_bcast(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), C * 0x55, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), C * 0x55, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+template <>
+struct Grp<4> {
+    // j is a constant after unrolling
+    static __device__ __forceinline__ double bc(double v, int j)
+    {
+        switch (j) {
+        case 0: return quad_bcast<0>(v);
+        case 1: return quad_bcast<1>(v);
+        case 2: return quad_bcast<2>(v);
+        default: return quad_bcast<3>(v);
+        }
+    }
+    static __device__ __forceinline__ double bc_dyn(double v, int j)
+    {
+        return __shfl(v, (int)(__lane_id() & 60u) + j);
+    }
+    static __device__ __forceinline__ int first(int v)
+    {
+        return __builtin_amdgcn_mov_dpp(v, 0, 0xf, 0xf, false);
+    }
+    static __device__ __forceinline__ bool all(bool p)
+    {
+        const unsigned long long b = __ballot(p);
+        return ((b >> (__lane_id() & 60u)) & 0xFull) == 0xFull;
+    }
+};
+
+// Row i of the packed lower triangle starts at i (i + 1) / 2.
+__host__ __device__ constexpr int tri(int i) { return i * (i + 1) / 2; }
 
 // Pairwise (tree) reductions of NM values: depth ceil(log2 NM) instead of NM.
 template <int NM>
@@ -757,6 +800,650 @@ struct Dense {
     }
 };
 
+// ---------------------------------------------------------------- one cell over G lanes
+// H as the bulk matrix-core sweeps leave it for the step pass: the lower triangle's 4 x 4 blocks
+// (R, C <= R), 16 consecutive doubles each, row-major; a last block row of one row (nm = 9, 25)
+// as that row alone.  A lane of the step pass then loads its rows as pairs of doubles, and the
+// lanes of a quad read whole 128-byte blocks.  Entries above the diagonal are not written.
+template <int NM>
+struct HBlock {
+    static constexpr bool kSingle = NM % 4 == 1;
+    static constexpr int kFull = 16 * tri(NM / 4);  // doubles of the whole blocks
+    static constexpr int kDoubles = kSingle ? kFull + NM + 1 : kFull;
+    static_assert(NM % 4 <= 1 && kDoubles <= NM * NM, "the state reserves nm * nm a cell");
+    static __host__ __device__ constexpr int at(int i, int j)
+    {
+        return kSingle && i == NM - 1 ? kFull + j
+                                      : 16 * (tri(i >> 2) + (j >> 2)) + 4 * (i & 3) + (j & 3);
+    }
+};
+
+// The step pass's algebra (not the reference-order mode's): element e of a cell's vectors sits
+// in register e / G of the cell's lane e % G, and so does row e of its matrix.  Every element
+// sees the operations of LaneVec<.., false> and Dense<.., false> in their order, so that a
+// cell's results are the tail's, which keeps one element per lane for its latency.
+//
+// The step pass is bound by instruction issue (dependent chains of the factorisation, of the
+// condition estimate's solves and of the reductions; a wave pays for an instruction whether or
+// not its lanes have rows left to update).  G = 4 up to nm = 16 puts 16 cells in a wave and the
+// solves' 4 x 4 blocks on whole quads; at nm = 25 a quad's rows would take 224 registers, so
+// G = 16 there, with four cells in a wave.
+template <int W>
+__device__ __forceinline__ int lane_plus(int v)  // from W lanes on, at lanes that are 0 mod 2W
+{
+    constexpr int ctrl = W == 1 ? 0xB1 : W == 2 ? 0x4E : 0x100 + W;  // quad_perm, row_shl
+    return __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, false);
+}
+template <int W>
+__device__ __forceinline__ double lane_plus(double v)
+{
+    return __hiloint2double(lane_plus<W>(__double2hiint(v)), lane_plus<W>(__double2loint(v)));
+}
+
+template <int NM, int G>
+struct Rows {
+    static constexpr int R = (NM + G - 1) / G;  // rows of a lane
+    static constexpr int NB = (NM + 3) / 4;     // 4 x 4 blocks
+    static constexpr bool kPad = NM % G != 0;   // the last row is not on every lane
+    // row e = G r + lane sits in L[at(r, 0)..], columns below width(r)
+    static constexpr int width(int r) { return G * (r + 1) < NM ? G * (r + 1) : NM; }
+    static constexpr int at(int r, int j) { return r * (r + 1) / 2 * G + j; }
+    static constexpr int kElems = at(R - 1, 0) + NM;
+    // Columns for the transposed solves, in LDS: slot (b, r) holds, for each of the cell's lanes,
+    // L(4 b + c, G r + lane), c = 0..3 (block b's rows at the columns of register r).
+    static constexpr int slots(int b) { return (4 * b + G - 1) / G; }
+    static constexpr int slot(int b, int r)
+    {
+        int o = r;
+        for (int k = 1; k < b; ++k)
+            o += slots(k);
+        return o;
+    }
+    static constexpr int kSlots = NB > 1 ? slot(NB, 0) : 1;
+    static constexpr int kLds = kSlots * 4 * kWave;  // doubles a wave
+
+    double L[kElems];
+    double tr[R][4], tc[R][4];  // row and column lane % 4 of the diagonal block's inverse
+
+    static __device__ __forceinline__ bool own(int r, int gl)
+    {
+        return !kPad || r + 1 < R || G * r + gl < NM;
+    }
+    static __device__ __forceinline__ double bc(const double (&x)[R], int e)
+    {
+        return Grp<G>::bc(x[e / G], e % G);
+    }
+    static __device__ __forceinline__ double bc_dyn(const double (&x)[R], int e)
+    {
+        double v = Grp<G>::bc_dyn(x[0], e % G);
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+            const double w = Grp<G>::bc_dyn(x[r], e % G);
+            v = e >= G * r ? w : v;
+        }
+        return v;
+    }
+    __device__ __forceinline__ double entry(int i, int j) const  // L(i, j) on every lane
+    {
+        return Grp<G>::bc(L[at(i / G, j)], i % G);
+    }
+
+    // ---- reductions over the cell's elements: the binary trees of tree_sum / tree_max over the
+    // element index, lanes first, then registers.  Absent elements hold the operation's identity
+    // (-0.0 for the sum: v + -0.0 is v for every v).
+    static __device__ __forceinline__ double sum(double (&v)[R])
+    {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            v[r] = v[r] + lane_plus<1>(v[r]);
+            v[r] = v[r] + lane_plus<2>(v[r]);
+            if constexpr (G == 16) {
+                v[r] = v[r] + lane_plus<4>(v[r]);
+                v[r] = v[r] + lane_plus<8>(v[r]);
+            }
+        }
+        const double s = tree_sum(v);
+        return G == 4 ? s : Grp<G>::bc(s, 0);
+    }
+    static __device__ __forceinline__ double max2(double a, double b) { return b > a ? b : a; }
+    static __device__ __forceinline__ double max(double (&v)[R])
+    {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            v[r] = max2(v[r], lane_plus<1>(v[r]));
+            v[r] = max2(v[r], lane_plus<2>(v[r]));
+            if constexpr (G == 16) {
+                v[r] = max2(v[r], lane_plus<4>(v[r]));
+                v[r] = max2(v[r], lane_plus<8>(v[r]));
+            }
+        }
+        return Grp<G>::bc(tree_max(v), 0);
+    }
+    static __device__ __forceinline__ double dasum(const double (&x)[R], int gl)
+    {
+        double v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            v[r] = own(r, gl) ? fabs(x[r]) : -0.0;
+        return sum(v);
+    }
+    static __device__ __forceinline__ double dot(const double (&x)[R], const double (&y)[R],
+                                                 int gl)
+    {
+        double v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            v[r] = own(r, gl) ? x[r] * y[r] : -0.0;
+        return sum(v);
+    }
+    template <int W>
+    static __device__ __forceinline__ void max_index_step(double &t, int &k)
+    {
+        const double to = lane_plus<W>(t);
+        const int ko = lane_plus<W>(k);
+        const bool take = to > t;
+        t = take ? to : t;
+        k = take ? ko : k;
+    }
+    static __device__ __forceinline__ int idamax(const double (&x)[R], int gl)
+    {
+        double t[R];
+        int k[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            t[r] = own(r, gl) ? fabs(x[r]) : -1.0;
+            k[r] = G * r + gl;
+            max_index_step<1>(t[r], k[r]);
+            max_index_step<2>(t[r], k[r]);
+            if constexpr (G == 16) {
+                max_index_step<4>(t[r], k[r]);
+                max_index_step<8>(t[r], k[r]);
+            }
+        }
+#pragma unroll
+        for (int w = 1; w < R; w *= 2)
+#pragma unroll
+            for (int i = 0; i + w < R; i += 2 * w)
+                if (t[i + w] > t[i]) {
+                    t[i] = t[i + w];
+                    k[i] = k[i + w];
+                }
+        return Grp<G>::first(k[0]);
+    }
+    static __device__ __forceinline__ double dnrm2(const double (&x)[R], int gl)
+    {
+        double v[R], t[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            v[r] = fabs(x[r]);
+            t[r] = own(r, gl) ? v[r] : -1.0;
+        }
+        const double scale = max(t);
+        if (!(scale > 0.0) || !isfinite(scale))
+            return scale;  // 0, inf or NaN
+        const double rs = 1.0 / scale;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const double q = v[r] * rs;
+            t[r] = own(r, gl) ? q * q : -0.0;
+        }
+        return scale * sqrt(sum(t));
+    }
+    // the reference BLAS's sequential form (LaneVec<NM>::dnrm2; the unbatched semantics' rtol)
+    static __device__ __forceinline__ double dnrm2_ref(const double (&x)[R])
+    {
+        double scale = 0.0, ssq = 1.0;
+#pragma unroll 1
+        for (int i = 0; i < NM; ++i) {
+            const double xi = bc_dyn(x, i);
+            const double a = fabs(xi);
+            const bool up = scale < a;
+            const double q = (up ? scale : a) / (up ? a : scale);
+            if (xi != 0.0) {
+                if (up) {
+                    ssq = 1.0 + ssq * (q * q);
+                    scale = a;
+                } else {
+                    ssq = ssq + q * q;
+                }
+            }
+        }
+        return scale * sqrt(ssq);
+    }
+
+    // ---- the matrix
+    __device__ __forceinline__ void load(const double *H, int gl)
+    {
+        typedef double du2 __attribute__((ext_vector_type(2), aligned(8)));
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int e = G * r + gl, b = e >> 2;
+            const bool single = HBlock<NM>::kSingle && e == NM - 1;
+            const double *row = H + (single ? HBlock<NM>::kFull : 16 * tri(b) + 4 * (e & 3));
+            const int step = single ? 4 : 16;
+#pragma unroll
+            for (int C = 0; 4 * C < width(r); ++C) {
+                const bool have = own(r, gl) && (G == 4 || C <= b);
+                if (4 * C + 3 < NM) {
+                    du2 v0 = {0.0, 0.0}, v1 = {0.0, 0.0};
+                    if (have) {
+                        v0 = *(const du2 *)(row + step * C);
+                        v1 = *(const du2 *)(row + step * C + 2);
+                    }
+                    L[at(r, 4 * C)] = v0.x;
+                    L[at(r, 4 * C + 1)] = v0.y;
+                    L[at(r, 4 * C + 2)] = v1.x;
+                    L[at(r, 4 * C + 3)] = v1.y;
+                } else {
+#pragma unroll
+                    for (int j = 4 * C; j < NM; ++j)
+                        L[at(r, j)] = have ? row[step * C + (j & 3)] : 0.0;
+                }
+            }
+        }
+    }
+
+    // The lane's own columns of the rows below its blocks, through the wave's LDS (sC, kLds
+    // doubles): the writer of row 4 b + c puts column t at place (t + c) mod 4 of t's quad, so
+    // that neither its stores nor the reads share banks.
+    __device__ __forceinline__ void store_columns(double *sC, int lane, int gl) const
+    {
+        wave_lds_sync();
+#pragma unroll
+        for (int b = 1; b < NB; ++b) {
+            const int c = gl & 3;
+            if ((G == 4 || (gl >> 2) == b % (G / 4)) && own(4 * b / G, gl)) {
+#pragma unroll
+                for (int t = 0; t < 4 * NB; ++t)
+                    if (t < 4 * b)
+                        sC[(slot(b, t / G) * 4 + c) * kWave + (lane - gl) + (t % G & ~3) +
+                           ((t + c) & 3)] = L[at(4 * b / G, t)];
+            }
+        }
+        wave_lds_sync();
+    }
+    // L(4 b + c, G r + lane), for lanes with G r + lane < 4 b and rows 4 b + c < nm
+    static __device__ __forceinline__ double column(const double *sC, int b, int r, int c,
+                                                    int lane)
+    {
+        return sC[(slot(b, r) * 4 + c) * kWave + (lane & ~3) + ((lane + c) & 3)];
+    }
+    // entry c of the lane's row within its own diagonal block (0 beyond nm)
+    __device__ __forceinline__ double own_block(int r, int c, int gl) const
+    {
+        double v = G * r + c < NM ? L[at(r, G * r + c)] : 0.0;
+        if constexpr (G == 16) {
+#pragma unroll
+            for (int k = 1; k < 4; ++k)
+                if (G * r + 4 * k < NM) {
+                    const double w = G * r + 4 * k + c < NM ? L[at(r, G * r + 4 * k + c)] : 0.0;
+                    v = (gl >> 2) == k ? w : v;
+                }
+        }
+        return v;
+    }
+
+    // utils_norm1 (the largest absolute row sum) of the symmetric matrix in L: each row's sum is
+    // a tree over the whole row, its part right of the diagonal block from the column slots
+    __device__ __forceinline__ double norm1(double *sC, int lane, int gl) const
+    {
+        store_columns(sC, lane, gl);
+        double rs[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int b = G == 4 ? r : (G * r + gl) >> 2;
+            double t[NM], dg[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                dg[c] = own_block(r, c, gl);
+#pragma unroll
+            for (int c = 1; c < 4; ++c)
+#pragma unroll
+                for (int l = 0; l < c; ++l) {
+                    const double v = Grp<4>::bc(dg[l], c);  // (c, l) of the block, for row l
+                    dg[c] = (gl & 3) == l ? v : dg[c];
+                }
+#pragma unroll
+            for (int j = 0; j < NM; ++j) {
+                const int C = j >> 2;
+                double v = 4 * C < width(r) ? L[at(r, j)] : 0.0;
+                if (G == 4 ? C == r : (G * r <= 4 * C && 4 * C < G * (r + 1)))
+                    v = C == b ? dg[j & 3] : v;
+                if (4 * C > G * r && C > 0)
+                    v = C > b ? column(sC, C, r, j & 3, lane) : v;
+                t[j] = fabs(v);
+            }
+            rs[r] = own(r, gl) ? tree_sum(t) : -1.0;
+            __builtin_amdgcn_sched_barrier(0);  // one row's entries in registers at a time
+        }
+        return fmax(max(rs), 0.0);
+    }
+
+    // Dense::cholesky_short.  Returns 0, or nonzero if a pivot was not positive.
+    __device__ __forceinline__ int cholesky(int gl)
+    {
+        int bad = 0;
+        cholesky_from<0>(gl, bad);
+        return bad;
+    }
+    template <int J>
+    __device__ __forceinline__ void cholesky_from(int gl, int &bad)
+    {
+        constexpr int rj = J / G, W = J > 0 ? J : 1;
+        double t[W], bj[W];
+#pragma unroll
+        for (int k = 0; k < J; ++k) {
+            t[k] = L[at(rj, k)] * L[at(rj, k)];
+            bj[k] = Grp<G>::bc(L[at(rj, k)], J % G);
+        }
+        const double ajj = Grp<G>::bc(L[at(rj, J)] - (J > 0 ? tree_sum(t) : 0.0), J % G);
+        if (!(ajj > 0.0))
+            bad = 1;
+        double q;
+        if (ajj > 1e-280 && ajj < 1e280) {  // far from the exponent range's ends
+            q = __builtin_amdgcn_rsq(ajj);
+            q = q * (1.5 - (0.5 * ajj) * (q * q));
+            q = q * (1.5 - (0.5 * ajj) * (q * q));
+        } else {
+            q = 1.0 / sqrt(ajj);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r >= rj && G * r + G - 1 > J) {  // a row below J
+#pragma unroll
+                for (int k = 0; k < J; ++k)
+                    t[k] = bj[k] * L[at(r, k)];
+                const double y = L[at(r, J)] - (J > 0 ? tree_sum(t) : 0.0);
+                if (r > rj || gl > J % G)
+                    L[at(r, J)] = q * y;
+            }
+            if (r == rj && gl == J % G)
+                L[at(rj, J)] = ajj * q;
+            // here, or the later rows' updates sink to their first use and hold the broadcasts
+            // of every column until then
+            if (r >= rj)
+                asm volatile("" : "+v"(L[at(r, J)]));
+        }
+        if constexpr (J + 1 < NM)
+            cholesky_from<J + 1>(gl, bad);
+    }
+
+    // Dense::build_columns and block_inverse
+    __device__ __forceinline__ void prepare_solves(double *sC, int lane, int gl)
+    {
+        store_columns(sC, lane, gl);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int l4 = gl & 3;
+            double dg[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                dg[c] = own_block(r, c, gl);
+                if (!own(r, gl))  // identity rows beyond nm
+                    dg[c] = c == l4 ? 1.0 : 0.0;
+            }
+            double djj = dg[0];
+#pragma unroll
+            for (int c = 1; c < 4; ++c)
+                djj = l4 == c ? dg[c] : djj;
+            const double dinv = 1.0 / djj;
+            double T[4][4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                T[i][i] = Grp<4>::bc(dinv, i);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int i = c + 1; i < 4; ++i) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int k = c; k < i; ++k)
+                        s = s + Grp<4>::bc(dg[k], i) * T[k][c];
+                    T[i][c] = -s * T[i][i];
+                }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                double vr = 0.0, vc = 0.0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (i == l4) {
+                        vr = (c <= i) ? T[i][c] : 0.0;
+                        vc = (c >= i) ? T[c][i] : 0.0;
+                    }
+                }
+                tr[r][c] = vr;
+                tc[r][c] = vc;
+            }
+        }
+    }
+
+    // x <- L^-1 x (Dense::trsv_ln_blocked)
+    __device__ __forceinline__ void trsv_ln(double (&x)[R], int gl) const
+    {
+        const int l4 = gl & 3;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int rb = 4 * b / G;
+            double xb[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                xb[c] = (4 * b + c < NM) ? bc(x, 4 * b + c) : 0.0;
+            double y = 0.0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const double yn = y + tr[rb][c] * xb[c];
+                y = c <= l4 ? yn : y;
+            }
+            if ((G == 4 || (gl >> 2) == b % (G / 4)) && own(rb, gl))
+                x[rb] = y;
+            if (b + 1 < NB) {
+                double yb[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    yb[c] = bc(x, 4 * b + c);
+#pragma unroll
+                for (int r = rb; r < R; ++r) {
+                    if (G * (r + 1) <= 4 * b + 4)
+                        continue;  // no row below the block
+                    double v = x[r];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        v = v - L[at(r, 4 * b + c)] * yb[c];
+                    if (G * r >= 4 * b + 4 || G * r + gl >= 4 * b + 4)
+                        x[r] = v;
+                }
+            }
+        }
+    }
+    // x <- L^-T x (Dense::trsv_lt_blocked)
+    __device__ __forceinline__ void trsv_lt(double (&x)[R], const double *sC, int lane,
+                                            int gl) const
+    {
+        const int l4 = gl & 3;
+#pragma unroll
+        for (int b = NB - 1; b >= 0; --b) {
+            const int rb = 4 * b / G;
+            double xb[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                xb[c] = (4 * b + c < NM) ? bc(x, 4 * b + c) : 0.0;
+            double y = 0.0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const double yn = y + tc[rb][c] * xb[c];
+                y = c >= l4 ? yn : y;
+            }
+            if ((G == 4 || (gl >> 2) == b % (G / 4)) && own(rb, gl))
+                x[rb] = y;
+            if (b > 0) {
+                double yb[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    yb[c] = (4 * b + c < NM) ? bc(x, 4 * b + c) : 0.0;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (G * r >= 4 * b)
+                        continue;  // no column left of the block
+                    double v = x[r];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (4 * b + c < NM)
+                            v = v - column(sC, b, r, c, lane) * yb[c];
+                    if (G * (r + 1) <= 4 * b || G * r + gl < 4 * b)
+                        x[r] = v;
+                }
+            }
+        }
+    }
+    // The factor into H's place, for potrs_lapack.
+    __device__ __forceinline__ void save(double *H, int gl) const
+    {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int j = 0; j < NM; ++j)
+                if (j < width(r) && own(r, gl) && j <= G * r + gl)
+                    H[HBlock<NM>::at(G * r + gl, j)] = L[at(r, j)];
+        __threadfence_block();
+    }
+    // Dense::potrs_lapack with the saved factor (the unbatched semantics; kept compact)
+    static __device__ __forceinline__ void potrs_lapack(double (&d)[R], const double *F, int gl)
+    {
+        auto put = [&](int e, double v) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                d[r] = G * r + gl == e ? v : d[r];
+        };
+#pragma unroll 1
+        for (int k = 0; k < NM; ++k) {
+            double dk = bc_dyn(d, k);
+            if (dk != 0.0) {
+                dk = dk * (1.0 / F[HBlock<NM>::at(k, k)]);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int e = G * r + gl;
+                    if (e > k && e < NM)
+                        d[r] = d[r] - dk * F[HBlock<NM>::at(e, k)];
+                }
+                put(k, dk);
+            }
+        }
+#pragma unroll 1
+        for (int i = NM - 1; i >= 0; --i) {
+            double temp = bc_dyn(d, i);
+#pragma unroll 1
+            for (int k = i + 1; k < NM; ++k)
+                temp = temp - F[HBlock<NM>::at(k, i)] * bc_dyn(d, k);
+            put(i, temp * (1.0 / F[HBlock<NM>::at(i, i)]));
+        }
+    }
+
+    // (max_i L_ii / min_i L_ii)^2 over the factor's diagonal (Dense::diag_ratio_sq)
+    __device__ __forceinline__ double diag_ratio_sq() const
+    {
+        double dmax = entry(0, 0), dmin = dmax;
+#pragma unroll
+        for (int i = 1; i < NM; ++i) {
+            const double v = entry(i, i);
+            dmax = fmax(dmax, v);
+            dmin = fmin(dmin, v);
+        }
+        const double q = dmax / dmin;
+        return q * q;
+    }
+
+    // Dense::pocon: dpocon('L') as dlacn2 (Higham 1988) over the blocked solves
+    __device__ __forceinline__ double pocon(double anorm, const double *sC, int lane, int gl) const
+    {
+        if (anorm == 0.0)
+            return 0.0;
+        double x[R];
+        int isgn[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            x[r] = own(r, gl) ? 1.0 / (double)NM : 0.0;
+            isgn[r] = 0;
+        }
+        auto signs = [&] {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (own(r, gl)) {
+                    x[r] = (x[r] >= 0.0) ? 1.0 : -1.0;
+                    isgn[r] = (x[r] >= 0.0) ? 1 : -1;
+                }
+        };
+        auto unit = [&](int e) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                x[r] = (G * r + gl == e) ? 1.0 : 0.0;
+        };
+        double est = 0.0;
+        int stage = 1, j2 = 0, iter = 0;
+        for (int guard = 0; guard < 16; ++guard) {
+            int z = 0;  // the columns are read from LDS each time, not kept in registers
+            if constexpr (NM > 9)
+                asm volatile("" : "+s"(z));
+            trsv_ln(x, gl);
+            trsv_lt(x, sC + z, lane, gl);
+            bool last = false;
+            if (stage & 1) {  // 1, 3, 5: a 1-norm
+                const double as = dasum(x, gl);
+                if (stage == 5) {
+                    const double temp = 2.0 * (as / (double)(3 * NM));
+                    if (temp > est)
+                        est = temp;
+                    break;
+                }
+                const double estold = est;
+                est = as;
+                if (stage == 1) {
+                    signs();
+                    stage = 2;
+                    continue;
+                }
+                bool same = true;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    same = same && (!own(r, gl) || (((x[r] >= 0.0) ? 1 : -1) == isgn[r]));
+                if (Grp<G>::all(same) || est <= estold) {
+                    last = true;
+                } else {
+                    signs();
+                    stage = 4;
+                    continue;
+                }
+            } else {  // 2, 4: the largest component
+                const int jlast = j2;
+                j2 = idamax(x, gl);
+                if (stage == 2) {
+                    iter = 2;
+                    unit(j2);
+                    stage = 3;
+                    continue;
+                }
+                if (bc_dyn(x, jlast) != fabs(bc_dyn(x, j2)) && iter < 5) {
+                    ++iter;
+                    unit(j2);
+                    stage = 3;
+                    continue;
+                }
+                last = true;
+            }
+            if (last) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int e = G * r + gl;
+                    x[r] = own(r, gl)
+                               ? ((e & 1) ? -1.0 : 1.0) * (1.0 + (double)e / (double)(NM - 1))
+                               : 0.0;
+                }
+                stage = 5;
+            }
+        }
+        return est != 0.0 ? (1.0 / est) / anorm : 0.0;
+    }
+};
+
 // ---------------------------------------------------------------- init pass
 // preProcess (optBatch.cpp:312-331 / opt.cpp:336-346) and the first worklist.
 template <int NM>
@@ -902,9 +1589,6 @@ struct ChunkStager {
     }
 };
 
-// Row i of the packed lower triangle starts at i (i + 1) / 2.
-__host__ __device__ constexpr int tri(int i) { return i * (i + 1) / 2; }
-
 // The chunk ordinate whose exponent and weight lane l computes in the tail's FP64 sweep.
 __device__ __forceinline__ int mfma_ordinate(int lane) { return lane; }
 
@@ -941,15 +1625,6 @@ __device__ __forceinline__ void chunk_mfma(const double *sMc, double wl, const d
             acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(wq * b1, b1, acc[2], 0, 0, 0);
         }
     }
-}
-
-// Lane C of the lane's quad (four consecutive lanes), on the vector unit.
-template <int C>
-__device__ __forceinline__ double quad_bcast(double v)
-{
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), C * 0x55, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), C * 0x55, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
 }
 
 // The bulk FP64 sweep of four cells a wave on V_MFMA_F64_4X4X4_4B_F64 (as fast per flop as the
@@ -1241,7 +1916,7 @@ __device__ __forceinline__ void store_H_ref(const RefEntries<NM> &E,
 
 // ---------------------------------------------------------------- sweep pass
 // A wavefront takes 4 cells (Quad); the block's 16 cells share every M chunk staged in LDS.
-// Writes H as its packed lower triangle, which is all the step pass reads.
+// Writes H's lower triangle in the step pass's layout (HBlock).
 template <int NM>
 __global__ __launch_bounds__(kBlock) void k_sweep(KParams P, const double *__restrict__ Mg,
                                                    const double *__restrict__ wg, State S,
@@ -1281,8 +1956,8 @@ __global__ __launch_bounds__(kBlock) void k_sweep(KParams P, const double *__res
         if (cell >= 0) {
             if ((lane & 0x33) == 0)
                 S.fdir[cell] = f;
-            double *H = S.H + (size_t)cell * NM * NM;
-            Q.each([&](int i, int j, double v) { H[tri(i) + j] = v; }, lane);
+            double *H = S.H + (size_t)cell * HBlock<NM>::kDoubles;
+            Q.each([&](int i, int j, double v) { H[HBlock<NM>::at(i, j)] = v; }, lane);
         }
     }
 }
@@ -1961,21 +2636,32 @@ __global__ __launch_bounds__(ColShape<NM>::kBlock) void k_sweep_cols(KParams P,
         if (g == 0 && cell >= 0)
             S.fdir[cell] = f * es;
         // H: accumulator k of lane l is the cell of column 4 (l >> 4) + k, pair 16 t + (l & 15)
+        int ck[4];
+        double sc[4];
+        bool ok[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int src = 4 * g + k;
-            const int ck = __shfl(cell, src);
-            const double sc = pair_scale(__shfl(es, src));
-            const bool ok = h16_range_ok(__shfl(wm, src));
-            if (ck >= 0) {
-                double *H = S.H + (size_t)ck * NM * NM;
+            ck[k] = __shfl(cell, src);
+            sc[k] = pair_scale(__shfl(es, src));
+            ok[k] = h16_range_ok(__shfl(wm, src));
+        }
 #pragma unroll
-                for (int t = 0; t < PT; ++t) {
-                    const int p = 16 * t + i16;
-                    if (p < PH::NP)
-                        H[p] = (p == 0 && !ok) ? __builtin_nan("") : (double)acc[t][k] * sc;
-                }
-            }
+        for (int t = 0; t < PT; ++t) {
+            const int p = 16 * t + i16;
+            int i = 0;  // the pair's row: p = tri(i) + j
+#pragma unroll
+            for (int q = 1; q < NM; ++q)
+                if (tri(q) >= 16 * t && tri(q) <= 16 * t + 15)
+                    i = p >= tri(q) ? q : i;
+                else if (tri(q) < 16 * t)
+                    i = q;
+            const int off = HBlock<NM>::at(i, p - tri(i));
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (p < PH::NP && ck[k] >= 0)
+                    S.H[(size_t)ck[k] * HBlock<NM>::kDoubles + off] =
+                        (p == 0 && !ok[k]) ? __builtin_nan("") : (double)acc[t][k] * sc[k];
         }
         // gradient: register r of lane l is the cell of column (l >> 4) + 4 r, moment
         // 16 t + (l & 15)
@@ -2186,9 +2872,9 @@ struct Cell {
     // in LDS or global memory; fdir = sum_q w_q e_q): either the Armijo test of a line-search
     // trial, or one Newton iteration of solveTheRest / optScaled.  sT: NM x (NM+1) doubles of
     // LDS for the transposed factor.  Returns 0 to continue, 1 converged, 2 ladder exhausted.
-    // H is not read when a line-search trial is rejected (it may then be null).  PACKED: H is
-    // the packed lower triangle in the FP64 phase too (the bulk sweeps' form).
-    template <bool EXACT, bool PACKED = false>
+    // H is not read when a line-search trial is rejected (it may then be null); in the mixed
+    // phase it is the packed lower triangle.
+    template <bool EXACT>
     __device__ __forceinline__ int advance(const KParams &P, const double *H, double fdir,
                                            const double *gm, double *sT, int lane)
     {
@@ -2218,12 +2904,10 @@ struct Cell {
         // ================================ one Newton iteration (solveTheRest)
         const bool mx = mixed(P);
         Dense<NM, EXACT, G> D;
-        if (PACKED || mx) {  // the row's part above the diagonal mirrored (the mixed phase
-                             // does not read it)
+        if (mx) {
 #pragma unroll
             for (int j = 0; j < NM; ++j)
-                D.row[j] = own && (j <= lane || !mx) ? H[j <= lane ? tri(lane) + j : tri(j) + lane]
-                                                     : 0.0;
+                D.row[j] = own && j <= lane ? H[tri(lane) + j] : 0.0;
         } else {
 #pragma unroll
             for (int j = 0; j < NM; ++j)
@@ -2393,16 +3077,374 @@ struct Cell {
     }
 };
 
+// Cell::load, advance<false> and store for the step pass, on the layout of Rows.  step()
+// returns 0 (state stored, the cell continues), 1 converged or 2 ladder exhausted.  MX: the
+// cells of the mixed-phase list, which take neither the condition estimate nor the ladder.
+// What the end of the iteration needs is read again there rather than held through the factor
+// and the estimate, whose registers two waves a SIMD leave no room beside.
+template <int NM, int G, bool MX>
+struct StepCell {
+    using RW = Rows<NM, G>;
+    static constexpr int R = RW::R;
+    double a[R], uu[R];
+    double err, gamma;
+    int tot, igam, reg, flags;
+
+    // still in the mixed phase
+    __device__ __forceinline__ bool mixed() const
+    {
+        return MX && !(flags & (C3D_FLAG_FP64_FALLBACK | C3D_FLAG_FP64_FINISH));
+    }
+
+    __device__ __forceinline__ int step(const KParams &P, const State &S, int c, double *sC,
+                                        int lane, int gl)
+    {
+        auto own = [&](int k) { return RW::own(k, gl); };
+        double *vb = S.vec + (size_t)c * kVec * NM;
+        double *sc = S.scal + (size_t)c * kScal;
+        int *in = S.ints + (size_t)c * kInt;
+        auto put = [&](int v, const double (&x)[R]) {
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                if (own(k))
+                    vb[v * NM + G * k + gl] = x[k];
+        };
+        auto get = [&](int v, int k) { return own(k) ? vb[v * NM + G * k + gl] : 0.0; };
+
+        const double fdir = S.fdir[c];
+        RW D;
+        double *H = S.H + (size_t)c * HBlock<NM>::kDoubles;
+        D.load(H, gl);
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            a[k] = get(kVa, k);
+            uu[k] = get(kVu, k);
+        }
+        double tls = sc[kStls], tprev = sc[kStprev], maxF;
+        err = sc[kSerr];
+        int iter = in[kIiter];
+        tot = in[kItot];
+        reg = in[kIreg];
+        flags = in[kIflags];
+        const int phase = in[kIphase];
+        const int maxIt = in[kImaxIt];
+
+        // The next trial of the backtracking search at step tls from x0 along x1, or its end
+        // (Cell::ls_next)
+        auto ls_next = [&](const double (&x0)[R], const double (&x1)[R]) {
+            const bool on = tls * maxF > DBL_EPSILON / 2;
+            if (!on)
+                tprev = 0.0;
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                a[k] = on ? (own(k) ? x0[k] + tls * x1[k] : 0.0) : x0[k];
+            if (gl == 0) {
+                sc[kStls] = tls;
+                sc[kStprev] = tprev;
+                in[kIphase] = on ? kPhaseLS : kPhaseH;
+            }
+            put(kVa, a);
+        };
+        if (phase == kPhaseLS) {
+            const double fNew = fdir - RW::dot(a, uu, gl);
+            if (fNew <= sc[kSf] + 1e-3 * tls * sc[kSgd]) {
+                tprev = tls;  // accepted; H of this sweep belongs to the new alpha
+            } else {
+                double x0[R], x1[R];
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    x0[k] = get(kVaOld, k);
+                    x1[k] = get(kVd, k);
+                }
+                maxF = sc[kSmaxF];
+                tls = 0.5 * tls;
+                ls_next(x0, x1);
+                return 0;
+            }
+        }
+        const double h00 = D.entry(0, 0);
+        // an H marked out of FP16's range: re-centre the shift and sweep again (Cell::advance)
+        if (MX && !(h00 == h00)) {
+            const double lf = log(fdir);
+            const double ns = (lf > -700.0 && lf < 700.0) ? lf : 0.0;
+            if (ns != sc[kSshift]) {
+                if (gl == 0) {
+                    sc[kSshift] = ns;
+                    sc[kStprev] = tprev;
+                    in[kIphase] = kPhaseH;
+                }
+                return 0;
+            }
+        }
+        // ================================ one Newton iteration (solveTheRest)
+        int maxItNow = maxIt;
+        if (!P.unbatched && reg == kNumReg - 1)
+            maxItNow = 10 * maxIt;
+        ++iter;
+        ++tot;
+        // fobjMnUseH; the mixed phase's sweep left the FP64 gradient moments in the g slot, which
+        // the FP64 phase fills here
+        auto gradient = [&](int k) { return get(kVg, k) - (own(k) ? uu[k] : 0.0); };
+        if constexpr (!MX) {
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                if (own(k))
+                    vb[kVg * NM + G * k + gl] = D.L[RW::at(k, 0)] / P.m0;
+        }
+        {
+            const double f = (MX ? fdir : h00 / (P.m0 * P.m0)) - RW::dot(a, uu, gl);
+            if (gl == 0)
+                sc[kSf] = f;
+        }
+        double norm = 0.0;
+        if (!MX)
+            norm = D.norm1(sC, lane, gl);
+        const int cholErr = D.cholesky(gl);
+        if (P.unbatched)
+            D.save(H, gl);
+        double condest = 0.0;
+        if (cholErr == 0) {
+            D.prepare_solves(sC, lane, gl);
+            condest = MX ? D.diag_ratio_sq() : 1.0 / D.pocon(norm, sC, lane, gl);
+        }
+        // The iteration starts over from a (and uu); rtol follows the (new) u.  What is not
+        // stored is set by the next iteration before it is read.
+        auto start_over = [&](double rtol) {
+            put(kVa, a);
+            if (gl == 0) {
+                sc[kStprev] = 1.0;
+                if (P.unbatched)  // opt.cpp:195, 240, 270
+                    sc[kSrtol] = rtol;
+                in[kIiter] = 0;
+                in[kItot] = tot;
+                in[kIgam] = 0;
+                in[kIflags] = flags;
+                in[kIphase] = kPhaseH;
+            }
+        };
+        double shift = 0.0;
+        if (MX) {
+            const bool stalled = tprev == 0.0 || iter >= min(maxItNow, P.mixedMaxIter);
+            const bool illCond = cholErr != 0 || !(condest <= P.mixedCondMax);
+            if ((stalled || illCond) && tot > 1 && err <= P.mixedSwitch) {
+                // FP64 Hessians continue from this iterate (Cell::advance)
+                flags |= C3D_FLAG_FP64_FINISH;
+                if (gl == 0) {
+                    sc[kStprev] = 1.0;
+                    in[kIflags] = flags;
+                    in[kIphase] = kPhaseH;
+                }
+                return 0;
+            }
+            if (illCond || stalled) {  // Cell::restart_fp64
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    a[k] = get(kVaIn, k);
+                    uu[k] = get(kVuOrig, k);
+                }
+                put(kVa0, a);
+                put(kVu, uu);
+                tot = 0;
+                flags = C3D_FLAG_FP64_FALLBACK;
+                if (gl == 0) {
+                    sc[kSerr] = 0.0;
+                    sc[kSgamma] = 0.0;
+                    sc[kSr] = 0.0;
+                    sc[kSrtol] = P.tol;
+                    sc[kSshift] = 0.0;
+                    in[kIreg] = 0;
+                    in[kImaxIt] = P.maxIter;
+                }
+                start_over(P.unbatched ? RW::dnrm2_ref(uu) * P.tol : 0.0);
+                return 0;
+            }
+            const double lf = log(fdir);  // shift of the sweeps from this iterate on
+            shift = (lf > -700.0 && lf < 700.0) ? lf : 0.0;
+        } else if (tot == 1 && (cholErr != 0 || condest > P.condHMax)) {
+            // isotropic restart, optBatch.cpp:208-218
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                a[k] = (k == 0 && gl == 0) ? P.isoAlpha0 : 0.0;
+                uu[k] = get(kVu, k);
+            }
+            put(kVa0, a);
+            flags |= C3D_FLAG_ISO_RESTART;
+            start_over(P.unbatched ? RW::dnrm2_ref(uu) * P.tol : 0.0);
+            return 0;
+        } else if (iter >= maxItNow || cholErr != 0 || tprev == 0.0 || condest > P.condHMax) {
+            gamma = sc[kSgamma];
+            if (reg == kNumReg - 1) {  // ladder, optBatch.cpp:222-248
+                igam = in[kIgam];
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    a[k] = get(kVa, k);
+                    uu[k] = get(kVu, k);
+                }
+                return 2;
+            }
+            ++reg;
+            const double r = kReg[reg];
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                uu[k] = (k == 0 && gl == 0) ? 1.0 : get(kVuOrig, k) * (1.0 - r);
+                a[k] = get(kVa0, k);
+            }
+            put(kVu, uu);
+            if (gl == 0) {
+                sc[kSr] = r;
+                in[kIreg] = reg;
+                if (P.unbatched && reg == kNumReg - 1)
+                    in[kImaxIt] = 10 * maxIt;
+            }
+            start_over(P.unbatched ? RW::dnrm2_ref(uu) * P.tol : 0.0);
+            return 0;
+        }
+        double g[R], d[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            a[k] = get(kVa, k);
+            uu[k] = get(kVu, k);
+            g[k] = gradient(k);
+            d[k] = g[k];
+        }
+        igam = in[kIgam];
+        if (P.unbatched) {
+            RW::potrs_lapack(d, H, gl);
+        } else {
+            D.trsv_ln(d, gl);
+            D.trsv_lt(d, sC, lane, gl);
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            d[k] = own(k) ? -d[k] : 0.0;
+        err = RW::dnrm2(g, gl);
+        gamma = det_exp(2.0 * RW::dasum(d, gl) * P.minf);
+        // the stopping test on the FP64 gradient, in both phases (optBatch.cpp:268)
+        const double rtol = sc[kSrtol];
+        if (err <= rtol && gamma <= P.tolGamma)
+            return 1;
+        if (err <= rtol && gamma > P.tolGamma)
+            ++igam;
+        if (MX && err <= P.mixedSwitch && condest > P.mixedFinishCond)
+            flags |= C3D_FLAG_FP64_FINISH;
+        // linesearch.cpp:29-54
+        double t[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            t[k] = own(k) ? fabs(d[k]) / (fabs(a[k]) + 1e-100) : -1.0;
+        maxF = fmax(RW::max(t), 0.0);
+        const double gd = RW::dot(g, d, gl);
+        tls = 1.0;
+        put(kVaOld, a);
+        put(kVd, d);
+        if (gl == 0) {
+            sc[kSmaxF] = maxF;
+            sc[kSgd] = gd;
+            sc[kSerr] = err;
+            sc[kSgamma] = gamma;
+            if (MX)
+                sc[kSshift] = shift;
+            in[kIiter] = iter;
+            in[kItot] = tot;
+            in[kIgam] = igam;
+            in[kIflags] = flags;
+        }
+        double x0[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            x0[k] = a[k];
+        ls_next(x0, d);
+        return 0;
+    }
+
+    // postProcess and the per-cell statistics (Cell::finish)
+    __device__ __forceinline__ void finish(const State &S, int done, int c, double *u_g,
+                                           double *alpha_g, c3d_cell_stats *stats, int *status,
+                                           int gl)
+    {
+        const double *sc = S.scal + (size_t)c * kScal;
+        const double u0 = sc[kSu0], r = sc[kSr];
+        if (done == 2)
+            flags |= C3D_FLAG_LADDER;
+        const double alphaScale = det_log(u0) * 2.0 * sqrt(M_PI);
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (RW::own(k, gl)) {
+                const int e = G * k + gl;
+                u_g[(size_t)c * NM + e] = uu[k] * u0;
+                alpha_g[(size_t)c * NM + e] = (e == 0) ? a[k] + alphaScale : a[k];
+            }
+        if (gl == 0) {
+            if (done == 2)
+                atomicOr(status, C3D_FLAG_LADDER);
+            if (stats) {
+                c3d_cell_stats s0{r, err, gamma, tot, igam, reg, flags};
+                stats[c] = s0;
+            }
+        }
+    }
+};
+
 // ---------------------------------------------------------------- step pass
-// One state-machine step per listed cell.  Orders up to M_3 (NM <= 16) take four cells per
-// wave, one per 16-lane row, so that the serial Cholesky / solve / condition-estimate chains
-// of four cells run side by side; larger orders take one cell per wave.  Two waves per SIMD
-// (at most 256 registers a lane) measured faster than one wave with no spills.
-template <int NM, bool EXACT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_step(KParams P, State S, Lists Lc, Lists Ln,
-                                                  double *u_g, double *alpha_g,
-                                                  c3d_cell_stats *stats, int *status,
-                                                  unsigned long long *sweepCount)
+// One state-machine step per listed cell with the sweep's H (HBlock layout): Cell::advance<false>
+// on the layout of Rows, the same decisions and bits.  One wave per block: waves run at their
+// own pace (a wave lasts as long as its slowest cell), and two fit a SIMD.  A spilled register
+// costs more here than an instruction: with about 200 of them the waves' scratch did not stay
+// in L2 and nm = 16 ran at the one-row-per-lane layout's speed.  Measured against that layout
+// (four cells a wave, one at nm = 25), step passes only: an M_2 step of 128^3 cells 29.2 -> 10.1
+// ms, the mixed M_3 closure of 2^20 cells 16.4 -> 6.7 ms, the FP64 one of 150001 cells 5.9 ->
+// 2.3 ms, the mixed M_4 closure of 40961 cells 7.5 -> 2.5 ms.
+constexpr int step_group(int nm) { return nm <= 16 ? 4 : 16; }
+
+template <int NM>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void k_step(
+    KParams P, State S, Lists Lc, Lists Ln, double *u_g, double *alpha_g, c3d_cell_stats *stats,
+    int *status, unsigned long long *sweepCount)
+{
+    constexpr int G = step_group(NM);
+    constexpr int kCells = kWave / G;
+    __shared__ double sC[Rows<NM, G>::kLds];
+    const int nWm = uniform_int(*Lc.nm);
+    const int nW = nWm + uniform_int(*Lc.nf);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && sweepCount) {  // [0] FP64 sweeps, [2] mixed
+        atomicAdd(sweepCount, (unsigned long long)(nW - nWm));
+        atomicAdd(sweepCount + 2, (unsigned long long)nWm);
+    }
+    C3D_BLOCK_APPENDER(app);
+    // waves of the mixed-phase list, then of the FP64 list
+    const int mixedBlocks = (nWm + kCells - 1) / kCells;
+    const int blocks = mixedBlocks + (nW - nWm + kCells - 1) / kCells;
+    for (int blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
+        // opaque, or what follows from the lane alone (LDS places, masks, offsets) is computed
+        // once before the loop, and spilled
+        int lane = threadIdx.x;
+        asm volatile("" : "+v"(lane));
+        const int gl = lane & (G - 1);
+        auto cells = [&](auto &&C, const int *W, int n, int first) {
+            const int slot = first * kCells + lane / G;
+            if (slot < n) {
+                const int c = W[slot];
+                const int done = C.step(P, S, c, sC, lane, gl);
+                if (done)
+                    C.finish(S, done, c, u_g, alpha_g, stats, status, gl);
+                else if (gl == 0)
+                    app.push(C.mixed(), c);
+            }
+        };
+        if (blk < mixedBlocks)
+            cells(StepCell<NM, G, true>(), Lc.Wm, nWm, blk);
+        else
+            cells(StepCell<NM, G, false>(), Lc.Wf, nW - nWm, blk - mixedBlocks);
+        app.flush(Ln, blk + gridDim.x >= blocks, kCells);
+    }
+}
+
+// The step pass in the reference's operation order (H row-major, both triangles): one cell per
+// 16-lane row up to nm = 16, per wave at nm = 25.
+template <int NM>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_step_ref(
+    KParams P, State S, Lists Lc, Lists Ln, double *u_g, double *alpha_g, c3d_cell_stats *stats,
+    int *status, unsigned long long *sweepCount)
 {
     constexpr int G = NM <= 16 ? 16 : kWave;
     constexpr int kCellsPerBlock = kBlock / G;
@@ -2426,8 +3468,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             Cell<NM, G> C;
             C.load(S, c, lane);
             const int done =
-                C.template advance<EXACT, !EXACT>(P, S.H + (size_t)c * NM * NM, S.fdir[c],
-                                          S.vec + (size_t)c * kVec * NM + kVg * NM, sT[grp], lane);
+                C.template advance<true>(P, S.H + (size_t)c * NM * NM, S.fdir[c],
+                                         S.vec + (size_t)c * kVec * NM + kVg * NM, sT[grp], lane);
             if (done) {
                 C.finish(done, c, u_g, alpha_g, stats, status, lane);
             } else {
@@ -3458,11 +4500,11 @@ hipError_t run_closure(c3d_ctx_s *ctx, const KParams &P, double *u, double *alph
         if (ev)
             (void)hipEventRecord(ev[2], s);
         if (ref)
-            hipLaunchKernelGGL((k_step<NM, true>), dim3(grid_cap(ctx, 16)), dim3(kBlock), 0, s,
-                               P, S, Lc, Ln, u, alpha, stats, ctx->d_status, cntBulk);
+            hipLaunchKernelGGL(k_step_ref<NM>, dim3(grid_cap(ctx, 16)), dim3(kBlock), 0, s, P, S,
+                               Lc, Ln, u, alpha, stats, ctx->d_status, cntBulk);
         else
-            hipLaunchKernelGGL((k_step<NM, false>), dim3(grid_cap(ctx, 16)), dim3(kBlock), 0,
-                               s, P, S, Lc, Ln, u, alpha, stats, ctx->d_status, cntBulk);
+            hipLaunchKernelGGL(k_step<NM>, dim3(grid_cap(ctx, 16)), dim3(kWave), 0, s, P, S, Lc,
+                               Ln, u, alpha, stats, ctx->d_status, cntBulk);
         if (ev)
             (void)hipEventRecord(ev[3], s);
         return hipSuccess;
