@@ -101,12 +101,13 @@ struct c3d_ctx_s {
     uint16_t *d_P16 = nullptr;  // the pair image (nm <= kPairMaxNm), nqPad / kChunk chunks
     double *d_R = nullptr;      // the row image (nm <= kPairMaxNm), nqPad / kChunk chunks
     double *d_M2 = nullptr;    // [nqPad][nm2]
-    double *d_beta = nullptr, *d_betaVal = nullptr, *d_pnOps = nullptr;
+    double *d_beta = nullptr, *d_betaVal = nullptr;
+    double *d_pnOps = nullptr;  // [6] operators, each transposed
     int32_t *d_betaColInd = nullptr, *d_betaRowPtr = nullptr;
     // control words
     int *d_status = nullptr;                  // OR of per-cell error flags since c3d_sync
     // scratch owned by the context, grown on demand
-    c3d::DevBuf ansatz, uOld, flux;
+    c3d::DevBuf ansatz, uOld;
     c3d::DevBuf closureState;  // per-cell Newton state, Hessians, worklists
     c3d::DevBuf statsPart;     // c3d_stats_summary's per-block partial sums
     c3d::Mlp mlp;
@@ -172,7 +173,8 @@ int mlp_set(c3d_ctx_s *ctx, const float *params, const float *norm);
 int mlp_get(c3d_ctx_s *ctx, float *params, float *norm);
 
 // grid.hip
-hipError_t launch_ghost_fill(int nx, int ny, int nz, int nm, double *u, hipStream_t s);
+hipError_t launch_ghost_fill(int nx, int ny, int nz, int nm, double *u, hipStream_t s,
+                             double *u2 = nullptr);
 hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *alpha,
                          double *A, int isPn, hipStream_t s);
 hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *A,
@@ -181,6 +183,9 @@ hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *
                           double theta, int fuseEuler, int zeroGhosts, hipStream_t s);
 hipError_t launch_flux_moment(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *u,
                               double *flux, double dx, double dy, double dz, hipStream_t s);
+hipError_t launch_moment_rk2(c3d_ctx_s *ctx, int nx, int ny, int nz, double *u, double *b,
+                             const double *sigmaT, const double *sigmaS, double dt, double dx,
+                             double dy, double dz, hipStream_t s);
 hipError_t launch_euler(int nx, int ny, int nz, int nm, double *u, const double *flux,
                         const double *sigmaT, const double *sigmaS, double dt, hipStream_t s);
 hipError_t launch_rk2(int nx, int ny, int nz, int nm, double *u, double *uOld, int kind,

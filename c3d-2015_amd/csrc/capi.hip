@@ -119,7 +119,14 @@ int finish_ctx(c3d_ctx_s *ctx)
     UP(d_betaVal, t.betaVal);
     UP(d_betaColInd, t.betaColInd);
     UP(d_betaRowPtr, t.betaRowPtr);
-    UP(d_pnOps, t.pnOps);
+    {
+        const size_t nm2 = (size_t)t.nm * t.nm;
+        // 16 doubles of padding: the moment flux reads whole runs
+        std::vector<double> opsT(t.pnOps.size() + 16, 0.0);
+        for (size_t e = 0; e < t.pnOps.size(); ++e)
+            opsT[e / nm2 * nm2 + e % t.nm * t.nm + e % nm2 / t.nm] = t.pnOps[e];
+        UP(d_pnOps, opsT);
+    }
 #undef UP
     if (e == hipSuccess)
         e = hipMalloc((void **)&ctx->d_sweepCount, 3 * sizeof(unsigned long long));
@@ -266,7 +273,7 @@ int c3d_destroy(c3d_ctx ctx)
     void *ptrs[] = {ctx->d_w, ctx->d_xi, ctx->d_eta, ctx->d_mu, ctx->d_M, ctx->d_MT,
                     ctx->d_wpad, ctx->d_P16, ctx->d_R, ctx->d_M2, ctx->d_beta, ctx->d_betaVal, ctx->d_pnOps, ctx->d_betaColInd,
                     ctx->d_betaRowPtr, ctx->d_sweepCount, ctx->d_status, ctx->ansatz.p,
-                    ctx->uOld.p, ctx->flux.p, ctx->closureState.p};
+                    ctx->uOld.p, ctx->closureState.p};
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);
@@ -715,12 +722,12 @@ int c3d_update(c3d_ctx ctx, int nx, int ny, int nz, double *u, double *alpha,
     const bool needAnsatz = solver == 1 || pnUseKinetic;
     if (e == hipSuccess && needAnsatz)
         e = grow(ctx->ansatz, ng * ctx->t.nq * sizeof(double));
-    if (e == hipSuccess && !needAnsatz)
-        e = grow(ctx->flux, ng * nm * sizeof(double));
     if (e != hipSuccess)
         return C3D_ERR_HIP;
-    double *uOld = (double *)ctx->uOld.p, *A = (double *)ctx->ansatz.p,
-           *flux = (double *)ctx->flux.p;
+    double *uOld = (double *)ctx->uOld.p, *A = (double *)ctx->ansatz.p;
+    if (!needAnsatz)
+        return hip_status(launch_moment_rk2(ctx, nx, ny, nz, u, uOld, sigmaT, sigmaS, dt, dx, dy,
+                                            dz, s));
     e = launch_rk2(nx, ny, nz, nm, u, uOld, 0, s);
     for (int st = 0; st < 2 && e == hipSuccess; ++st) {
         e = launch_ghost_fill(nx, ny, nz, nm, u, s);
@@ -737,10 +744,6 @@ int c3d_update(c3d_ctx ctx, int nx, int ny, int nz, double *u, double *alpha,
             if (e == hipSuccess)
                 e = launch_stencil(ctx, nx, ny, nz, A, nullptr, u, sigmaT, sigmaS, dt, dx, dy, dz,
                                    theta, 1, 0, s);
-        } else if (!pnUseKinetic) {
-            e = launch_flux_moment(ctx, nx, ny, nz, u, flux, dx, dy, dz, s);
-            if (e == hipSuccess)
-                e = launch_euler(nx, ny, nz, nm, u, flux, sigmaT, sigmaS, dt, s);
         } else {
             e = launch_ansatz(ctx, nx, ny, nz, u, A, 1, s);
             if (e == hipSuccess)

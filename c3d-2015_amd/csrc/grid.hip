@@ -6,7 +6,9 @@
 //   k_stencil      limited upwind differences, sum_q m_q (Fx/dx+Fy/dy+Fz/dz), optionally
 //                  fused with the Euler stage             flux_kinetic.cpp:45-60, 126-196,
 //                                                        update.cpp:21-37
-//   k_flux_moment  P_N Fromm flux with half-range operators  flux_moment.cpp:30-104
+//   k_moment_stage P_N Fromm flux with half-range operators, alone or with the Euler stage
+//                  and the RK2 average                    flux_moment.cpp:30-104,
+//                                                        update.cpp:21-37, 268-274
 //   k_euler        Euler stage with isotropic scattering update.cpp:21-37
 //   k_rk2          uOld <- u / u <- (u + uOld)/2          update.cpp:206-212, 268-274
 //   k_make_batch   synthetic closure batch (SplitMix64 counter RNG)
@@ -40,8 +42,44 @@ struct Grid {
 
 Grid make_grid(int nx, int ny, int nz) { return Grid{nx, ny, nz, nx + 4, ny + 4, nz + 4}; }
 
+// ---------------------------------------------------------------- tiling of the interior
+// The stencil kernels give a block kTB consecutive cells of one x-plane's flattened (y, z)
+// interior, and order the blocks so that what one XCD has in flight is compact: block b goes
+// to XCD b % 8, so XCD x takes the x-th eighth of an order that walks strips of kStrip such
+// chunks along x.  A strip's planes are then fetched into that XCD's L2 once and reused by
+// the four planes after them; dealing consecutive chunks over the XCDs instead makes every
+// L2 fetch its own copy of the y and x neighbours.
+constexpr int kXcd = 8;
+constexpr int kStrip = 16;
+__host__ __device__ __forceinline__ int64_t plane_chunks(const Grid &G)
+{
+    return ((int64_t)G.ny * G.nz + kTB - 1) / kTB;
+}
+unsigned tile_blocks(const Grid &G)
+{
+    return (unsigned)((plane_chunks(G) * G.nx + kXcd - 1) / kXcd * kXcd);
+}
+struct Tile {
+    int i;      // x index of the block's plane, ghosts counted
+    int64_t p;  // first cell of the flattened interior plane
+};
+__device__ __forceinline__ bool tile_of(const Grid &G, Tile &t)
+{
+    const int64_t nP = plane_chunks(G), total = nP * G.nx;
+    const int64_t b = (int64_t)(blockIdx.x % kXcd) * (gridDim.x / kXcd) + blockIdx.x / kXcd;
+    if (b >= total)
+        return false;
+    const int64_t strip = b / (kStrip * (int64_t)G.nx);
+    const int64_t rem = b - strip * kStrip * G.nx;
+    const int64_t width = nP - strip * kStrip < kStrip ? nP - strip * kStrip : kStrip;
+    t.i = 2 + (int)(rem / width);
+    t.p = (strip * kStrip + rem % width) * kTB;
+    return true;
+}
+
 // ---------------------------------------------------------------- ghost fill
-__global__ void k_ghost_fill(Grid G, int nm, double *u)
+// u2, if not null, receives the same ghosts
+__global__ void k_ghost_fill(Grid G, int nm, double *u, double *u2)
 {
     // three slab families of 2 x 2 x (face area) cells, each copies nm moments
     const int64_t ax = (int64_t)2 * G.ny * G.nz, ay = (int64_t)2 * G.nx * G.nz,
@@ -90,7 +128,10 @@ __global__ void k_ghost_fill(Grid G, int nm, double *u)
                 src = G.idx(i, j, 2 + l);
             }
         }
-        u[dst * nm + m] = u[src * nm + m];
+        const double v = u[src * nm + m];
+        u[dst * nm + m] = v;
+        if (u2)
+            u2[dst * nm + m] = v;
     }
 }
 
@@ -265,67 +306,204 @@ __global__ void k_zero_ghost_flux(Grid G, int nm, double *flux)
 }
 
 // -------------------------------------------------------------- moment flux
-template <int NM>
-__global__ __launch_bounds__(kTB) void k_flux_moment(Grid G, const double *__restrict__ u,
-                                                      double *flux,
-                                                      const double *__restrict__ ops, double dx,
-                                                      double dy, double dz)
+enum : int { kMomFlux = 0, kMomStage1 = 1, kMomStage2 = 2 };
+
+__device__ __forceinline__ void wave_lds_sync()
 {
-    __shared__ double sO[6 * NM * NM];
-    for (int e = threadIdx.x; e < 6 * NM * NM; e += kTB)
-        sO[e] = ops[e];
-    __syncthreads();
-    const int64_t ni = (int64_t)G.nx * G.ny * G.nz;
-    const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
-    if (t >= ni)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ long long uniform_i64(long long v)
+{
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)(v & 0xffffffffll));
+    const int hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
+    return ((long long)hi << 32) | lo;
+}
+
+// operators are read kOpRun doubles at a time (the table is padded by as many)
+constexpr int kOpRun = 16;
+typedef double op8 __attribute__((ext_vector_type(8), aligned(8)));
+typedef double op4 __attribute__((ext_vector_type(4), aligned(8)));
+struct OpRun {
+    op8 lo, hi;
+};
+
+// One thread per interior cell.  Bound by the vector unit (six NM x NM products without FMA
+// contraction) and, close behind, by HBM.  A lane that reads its own cell's moments touches a
+// cache line of its own per load (36 lines a load at nm = 9, which bound the kernel), so each
+// wave reads the 64 cells of a stencil offset as one contiguous run, forms the differences on
+// the runs (they are elementwise) and turns only those to a cell per lane through its own LDS
+// rows.  opsT holds the operators' columns: uniform over the wave, they come as scalar
+// operands (broadcast reads from LDS would take twice the vector unit's time), a run of them
+// at a time, the next run's loads in flight while one is used.
+//   kMomFlux    dst = flux
+//   kMomStage1  dst = Euler(src, flux(src))
+//   kMomStage2  dst = (Euler(src, flux(src)) + dst) / 2
+// so that a two-stage step (u -> b, b -> u) neither copies u nor stores a flux.  Measured at
+// 128^3, nm = 9: a step 447 us, against 1272 with flux, Euler, copy and average apart.
+// P2: every spacing a power of two (division is multiplication by the exact reciprocal).
+template <int NM, int KIND, bool P2>
+__global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(NM <= 9 ? 3 : 1))) void k_moment_stage(Grid G, const double *__restrict__ src,
+                                                       double *dst,
+                                                       const double *__restrict__ opsT, double dx,
+                                                       double dy, double dz, double dt,
+                                                       const double *__restrict__ sigT,
+                                                       const double *__restrict__ sigS)
+{
+    constexpr int NMS = NM | 1;  // odd row stride: no bank conflicts reading a row per lane
+    __shared__ double sB[kTB / kWave][kWave * NMS];
+    __shared__ double sD[kTB / kWave][KIND == kMomFlux ? 1 : 2 * kWave];
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    double *const buf = sB[wv];
+    Tile T;
+    if (!tile_of(G, T))
         return;
-    const int k = 2 + (int)(t % G.nz);
-    const int j = 2 + (int)((t / G.nz) % G.ny);
-    const int i = 2 + (int)(t / ((int64_t)G.nz * G.ny));
-    const size_t c = G.idx(i, j, k);
-    const size_t strides[3] = {(size_t)G.NY * G.NZ, (size_t)G.NZ, 1};
-    const double hs[3] = {dx, dy, dz};
+    // lanes past the plane's end work on its last cell and write nothing
+    const int64_t np = (int64_t)G.ny * G.nz;
+    const int64_t p = T.p + threadIdx.x;
+    const bool have = p < np;
+    const int64_t pc = have ? p : np - 1;
+    const size_t c = G.idx(T.i, 2 + (int)(pc / G.nz), 2 + (int)(pc % G.nz));
+    const size_t c0 = (size_t)uniform_i64((long long)c);
+    // element lane + 64 k of the wave's run: its place in memory, in bytes from the first cell's
+    // moments (64 interior cells lie within a few rows or, where the rows are short, planes)
+    unsigned rel[NM];
+    const int crel = (int)(c - c0);
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
+        const int e = lane + kWave * k, l = e / NM;
+        rel[k] = 8u * (unsigned)(__shfl(crel, l) * NM + (e - l * NM));
+    }
+    auto el = [](const double *a, unsigned o) { return *(const double *)((const char *)a + o); };
+    auto place = [&](int k) {  // the same element in LDS
+        const int e = lane + kWave * k, l = e / NM;
+        return NM == NMS ? e : l * NMS + (e - l * NM);
+    };
+    auto run = [&](ptrdiff_t off) { return src + ((ptrdiff_t)c0 + off) * NM; };
     double out[NM];
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-        out[m] = 0.0;
-#pragma unroll
+#pragma unroll(NM <= 4 ? 3 : 1)
     for (int ax = 0; ax < 3; ++ax) {
-        const size_t s = strides[ax];
-        const double *um2 = u + (c - 2 * s) * NM, *um1 = u + (c - s) * NM, *u0 = u + c * NM,
-                     *up1 = u + (c + s) * NM, *up2 = u + (c + 2 * s) * NM;
-        const double *Op = sO + (2 * ax) * NM * NM, *Om = sO + (2 * ax + 1) * NM * NM;
-        double temp[NM], F[NM];
+        const ptrdiff_t s = ax == 0 ? (ptrdiff_t)G.NY * G.NZ : (ax == 1 ? (ptrdiff_t)G.NZ : 1);
+        const double h = ax == 0 ? dx : (ax == 1 ? dy : dz);
+        const double *O = opsT + (2 * ax) * NM * NM;
+        const double *a0 = run(0), *ap1 = run(s), *ap2 = run(2 * s), *am1 = run(-s),
+                     *am2 = run(-2 * s);
+        double tm[NM], F[NM];
+        auto put_tm = [&] {
+            wave_lds_sync();
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-            temp[m] = 0.25 * up1[m] + 0.75 * u0[m] - 1.25 * um1[m] + 0.25 * um2[m];
+            for (int k = 0; k < NM; ++k)
+                buf[place(k)] = tm[k];
+            wave_lds_sync();
+        };
+        wave_lds_sync();
 #pragma unroll
-        for (int r = 0; r < NM; ++r) {
-            double b = 0.0;
-#pragma unroll
-            for (int q = 0; q < NM; ++q)
-                b += Op[r * NM + q] * temp[q];
-            F[r] = b;
+        for (int k = 0; k < NM; ++k) {
+            const double up1 = el(ap1, rel[k]), u0 = el(a0, rel[k]), um1 = el(am1, rel[k]);
+            buf[place(k)] = 0.25 * up1 + 0.75 * u0 - 1.25 * um1 + 0.25 * el(am2, rel[k]);
+            tm[k] = -0.25 * el(ap2, rel[k]) + 1.25 * up1 - 0.75 * u0 - 0.25 * um1;
         }
+        wave_lds_sync();
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-            temp[m] = -0.25 * up2[m] + 1.25 * up1[m] - 0.75 * u0[m] - 0.25 * um1[m];
-#pragma unroll
-        for (int r = 0; r < NM; ++r) {
-            double b = F[r];
+        for (int i = 0; i < NM; ++i)
+            F[i] = 0.0;
+        if constexpr (NM <= 16) {
+            double t[NM];
 #pragma unroll
             for (int q = 0; q < NM; ++q)
-                b += Om[r * NM + q] * temp[q];
-            F[r] = b;
+                t[q] = buf[lane * NMS + q];
+            put_tm();
+#pragma unroll
+            for (int q = 0; q < NM; ++q)
+                tm[q] = buf[lane * NMS + q];
+            // element e of the stream of both operators' columns: row e % NM, column e / NM
+            constexpr int nOp = 2 * NM * NM, nRun = (nOp + kOpRun - 1) / kOpRun;
+            OpRun cur = *(const OpRun *)O, nxt = cur;
+#pragma unroll
+            for (int r = 0; r < nRun; ++r) {
+                // scalar loads return in any order, so a wait is for all of them: wait for
+                // this run here, before the next one's loads are issued
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" ::"s"(cur.lo), "s"(cur.hi));
+                if (r + 1 < nRun)
+                    nxt = *(const OpRun *)(O + (r + 1) * kOpRun);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < kOpRun; ++j) {
+                    const int e = r * kOpRun + j, q = e / NM, i = e % NM;
+                    if (e < nOp)
+                        F[i] += (j < 8 ? cur.lo[j & 7] : cur.hi[j & 7]) *
+                                (q < NM ? t[q % NM] : tm[q % NM]);
+                }
+                cur = nxt;
+            }
+        } else {  // two runs to a column, columns in a loop
+            static_assert(NM <= 16 || NM == 25, "runs of 13 and 12");
+            auto apply = [&](const double *Oc) {
+                op8 a8 = *(const op8 *)Oc;
+                op4 a4 = *(const op4 *)(Oc + 8);
+                double a1 = Oc[12], tn = buf[lane * NMS];
+#pragma unroll 1
+                for (int q = 0; q < NM; ++q) {
+                    const double t = tn;
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" ::"s"(a8), "s"(a4), "s"(a1), "v"(t));
+                    const op8 b8 = *(const op8 *)(Oc + 13);
+                    const op4 b4 = *(const op4 *)(Oc + 21);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < 13; ++i)
+                        F[i % NM] += (i < 8 ? a8[i & 7] : (i < 12 ? a4[i & 3] : a1)) * t;
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" ::"s"(b8), "s"(b4));
+                    Oc += NM;  // past the last column: the next operator's, or the padding
+                    a8 = *(const op8 *)Oc;
+                    a4 = *(const op4 *)(Oc + 8);
+                    a1 = Oc[12];
+                    tn = buf[lane * NMS + (q + 1 < NM ? q + 1 : q)];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 13; i < 25; ++i)
+                        F[i % NM] += (i < 21 ? b8[(i - 13) & 7] : b4[(i - 21) & 3]) * t;
+                }
+            };
+            apply(O);
+            put_tm();
+            apply(O + NM * NM);
         }
         // flux = xF/dx + yF/dy + zF/dz, accumulated left to right
+        const double rh = 1.0 / h;
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-            out[m] = (ax == 0) ? F[m] / hs[0] : out[m] + F[m] / hs[ax];
+        for (int m = 0; m < NM; ++m) {
+            const double t = P2 ? F[m] * rh : F[m] / h;
+            out[m] = ax == 0 ? t : out[m] + t;
+        }
+    }
+    wave_lds_sync();
+    if constexpr (KIND != kMomFlux) {  // the Euler factors of the lane's cell, update.cpp:28-35
+        const double st = sigT[c], ss = sigS[c];
+        sD[wv][2 * lane] = 1.0 + dt * ss - dt * st;
+        sD[wv][2 * lane + 1] = 1.0 - dt * st;
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m)
-        flux[c * NM + m] = out[m];
+        buf[lane * NMS + m] = out[m];
+    wave_lds_sync();
+    // the lanes that have a cell are the first of the wave, and so are their elements
+    const int nHave = __popcll(__ballot(have)) * NM;
+    double *const at = dst + c0 * NM;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
+        const int e = lane + kWave * k, l = e / NM;
+        double v = buf[place(k)];
+        if constexpr (KIND != kMomFlux)
+            v = el(run(0), rel[k]) * sD[wv][2 * l + (e - l * NM ? 1 : 0)] - dt * v;
+        if constexpr (KIND == kMomStage2)
+            v = 0.5 * (v + el(at, rel[k]));
+        if (e < nHave)
+            *(double *)((char *)at + rel[k]) = v;
+    }
 }
 
 // -------------------------------------------------------------------- euler
@@ -498,12 +676,12 @@ unsigned blocks_for(int64_t n, int tb = kTB, int64_t cap = 1 << 20)
 
 }  // namespace
 
-hipError_t launch_ghost_fill(int nx, int ny, int nz, int nm, double *u, hipStream_t s)
+hipError_t launch_ghost_fill(int nx, int ny, int nz, int nm, double *u, hipStream_t s, double *u2)
 {
     Grid G = make_grid(nx, ny, nz);
     int64_t total = ((int64_t)2 * ny * nz + (int64_t)2 * nx * nz + (int64_t)2 * nx * ny) * 2 * nm;
     hipLaunchKernelGGL(k_ghost_fill, dim3(blocks_for(total, 256, 65536)), dim3(256), 0, s, G,
-                       nm, u);
+                       nm, u, u2);
     return hipGetLastError();
 }
 
@@ -566,20 +744,56 @@ hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *
     return hipGetLastError();
 }
 
+namespace {
+template <int KIND>
+hipError_t launch_moment_stage(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *src,
+                               double *dst, const double *sigmaT, const double *sigmaS, double dt,
+                               double dx, double dy, double dz, hipStream_t s)
+{
+    Grid G = make_grid(nx, ny, nz);
+    const bool p2 = exact_reciprocal(dx) && exact_reciprocal(dy) && exact_reciprocal(dz);
+    dim3 grid(tile_blocks(G));
+#define C3D_MOMENT(NMV)                                                                        \
+    if (p2)                                                                                    \
+        hipLaunchKernelGGL((k_moment_stage<NMV, KIND, true>), grid, dim3(kTB), 0, s, G, src,   \
+                           dst, ctx->d_pnOps, dx, dy, dz, dt, sigmaT, sigmaS);                 \
+    else                                                                                       \
+        hipLaunchKernelGGL((k_moment_stage<NMV, KIND, false>), grid, dim3(kTB), 0, s, G, src,  \
+                           dst, ctx->d_pnOps, dx, dy, dz, dt, sigmaT, sigmaS)
+    switch (ctx->t.nm) {
+    case 4: C3D_MOMENT(4); break;
+    case 9: C3D_MOMENT(9); break;
+    case 16: C3D_MOMENT(16); break;
+    case 25: C3D_MOMENT(25); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef C3D_MOMENT
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_flux_moment(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *u,
                               double *flux, double dx, double dy, double dz, hipStream_t s)
 {
-    Grid G = make_grid(nx, ny, nz);
-    const int64_t ni = (int64_t)nx * ny * nz;
-    dim3 grid(blocks_for(ni, kTB, INT32_MAX));
-    switch (ctx->t.nm) {
-    case 4: hipLaunchKernelGGL(k_flux_moment<4>, grid, dim3(kTB), 0, s, G, u, flux, ctx->d_pnOps, dx, dy, dz); break;
-    case 9: hipLaunchKernelGGL(k_flux_moment<9>, grid, dim3(kTB), 0, s, G, u, flux, ctx->d_pnOps, dx, dy, dz); break;
-    case 16: hipLaunchKernelGGL(k_flux_moment<16>, grid, dim3(kTB), 0, s, G, u, flux, ctx->d_pnOps, dx, dy, dz); break;
-    case 25: hipLaunchKernelGGL(k_flux_moment<25>, grid, dim3(kTB), 0, s, G, u, flux, ctx->d_pnOps, dx, dy, dz); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return launch_moment_stage<kMomFlux>(ctx, nx, ny, nz, u, flux, nullptr, nullptr, 0.0, dx, dy,
+                                         dz, s);
+}
+
+// one SSP-RK2 step of the P_N equations with the moment flux; b: a grid's worth of scratch
+hipError_t launch_moment_rk2(c3d_ctx_s *ctx, int nx, int ny, int nz, double *u, double *b,
+                             const double *sigmaT, const double *sigmaS, double dt, double dx,
+                             double dy, double dz, hipStream_t s)
+{
+    hipError_t e = launch_ghost_fill(nx, ny, nz, ctx->t.nm, u, s);
+    if (e == hipSuccess)
+        e = launch_moment_stage<kMomStage1>(ctx, nx, ny, nz, u, b, sigmaT, sigmaS, dt, dx, dy, dz,
+                                            s);
+    if (e == hipSuccess)  // the step leaves u with the second stage's ghosts
+        e = launch_ghost_fill(nx, ny, nz, ctx->t.nm, b, s, u);
+    if (e == hipSuccess)
+        e = launch_moment_stage<kMomStage2>(ctx, nx, ny, nz, b, u, sigmaT, sigmaS, dt, dx, dy, dz,
+                                            s);
+    return e;
 }
 
 hipError_t launch_euler(int nx, int ny, int nz, int nm, double *u, const double *flux,
