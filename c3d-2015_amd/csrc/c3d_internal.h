@@ -95,6 +95,9 @@ struct c3d_ctx_s {
     int nqPad = 0;  // nq rounded up to kChunk
     // device tables
     double *d_w = nullptr, *d_xi = nullptr, *d_eta = nullptr, *d_mu = nullptr;
+    double *d_ord = nullptr;   // [nq + 2][4 + nm], rows (xi, eta, mu, w, M's row); two zero rows
+    int32_t *d_sgn = nullptr;  // [nq + 8], bits 0..2: xi, eta, mu > 0
+    int *d_wild = nullptr;     // the ansatz holds a NaN or a huge value (grid.hip)
     double *d_M = nullptr;     // [nqPad][nm], rows >= nq zero
     double *d_MT = nullptr;    // [nm][nqPad], the transpose of d_M
     double *d_wpad = nullptr;  // [nqPad], entries >= nq zero

@@ -96,6 +96,24 @@ int finish_ctx(c3d_ctx_s *ctx)
         UP(d_MT, MTp);
     }
     UP(d_wpad, wp);
+    {
+        // the flux kernels' ordinate table (grid.hip), padded for their loads ahead of use
+        const size_t row = 4 + (size_t)t.nm;
+        std::vector<double> ord((t.nq + 2) * row, 0.0);
+        std::vector<int32_t> sgn(t.nq + 8, 0);
+        for (int q = 0; q < t.nq; ++q) {
+            const double dir[3] = {t.xi[q], t.eta[q], t.mu[q]};
+            double *r = ord.data() + q * row;
+            for (int a = 0; a < 3; ++a) {
+                r[a] = dir[a];
+                sgn[q] |= (dir[a] > 0) << a;
+            }
+            r[3] = t.w[q];
+            std::memcpy(r + 4, t.M.data() + (size_t)q * t.nm, t.nm * sizeof(double));
+        }
+        UP(d_ord, ord);
+        UP(d_sgn, sgn);
+    }
     if (t.nm <= kPairMaxNm) {
         std::vector<uint16_t> img;
         pair_image(t, ctx->nqPad, img);
@@ -132,6 +150,8 @@ int finish_ctx(c3d_ctx_s *ctx)
         e = hipMalloc((void **)&ctx->d_sweepCount, 3 * sizeof(unsigned long long));
     if (e == hipSuccess)
         e = hipMalloc((void **)&ctx->d_status, sizeof(int));
+    if (e == hipSuccess)
+        e = hipMalloc((void **)&ctx->d_wild, sizeof(int));
     if (e == hipSuccess)
         e = hipMemset(ctx->d_status, 0, sizeof(int));
     if (e == hipSuccess)
@@ -272,7 +292,7 @@ int c3d_destroy(c3d_ctx ctx)
         return C3D_OK;
     void *ptrs[] = {ctx->d_w, ctx->d_xi, ctx->d_eta, ctx->d_mu, ctx->d_M, ctx->d_MT,
                     ctx->d_wpad, ctx->d_P16, ctx->d_R, ctx->d_M2, ctx->d_beta, ctx->d_betaVal, ctx->d_pnOps, ctx->d_betaColInd,
-                    ctx->d_betaRowPtr, ctx->d_sweepCount, ctx->d_status, ctx->ansatz.p,
+                    ctx->d_betaRowPtr, ctx->d_sweepCount, ctx->d_status, ctx->d_wild, ctx->d_ord, ctx->d_sgn, ctx->ansatz.p,
                     ctx->uOld.p, ctx->closureState.p};
     for (void *p : ptrs)
         if (p)

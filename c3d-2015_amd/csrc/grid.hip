@@ -18,6 +18,7 @@
 // A[q*Ng + cell], so every stencil load of a wavefront is one contiguous segment.
 // Every expression keeps the reference's evaluation order (no FMA contraction), so the
 // results match the CPU code bit for bit whenever the exponentials agree.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 
@@ -136,38 +137,81 @@ __global__ void k_ghost_fill(Grid G, int nm, double *u, double *u2)
 }
 
 // ------------------------------------------------------------------- ansatz
-// One thread per cell (all cells, ghosts included), M staged through LDS 64 ordinates at
-// a time; the ansatz argument keeps flux_kinetic.cpp:23-24's sequential order.
-template <int NM>
-__global__ __launch_bounds__(kTB) void k_ansatz(int64_t ng, int nq, const double *__restrict__ M,
-                                                 const double *__restrict__ alpha, double *A,
-                                                 int isPn)
+// Row q of the ordinate table the flux kernels read as scalar operands: xi, eta, mu, w, then
+// M's row.  Its loads are issued a piece ahead of their use: scalar loads return in any order,
+// so a wait is for all of them, and use_s() waits for one piece before the next is issued.
+constexpr int ord_row(int nm) { return 4 + nm; }
+__device__ __forceinline__ void use_s(double x) { asm volatile("" ::"s"(x)); }
+template <int N>
+__device__ __forceinline__ void use_s(const double (&x)[N])
 {
-    __shared__ double sM[kChunk * NM];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        use_s(x[i]);
+}
+
+// One thread per cell (all cells, ghosts included) and blockIdx.y's share of the ordinates;
+// the ansatz argument keeps flux_kinetic.cpp:23-24's sequential order.  Bound by the vector
+// unit (the argument without FMA contraction, then exp) and the store of A.  M's rows are
+// uniform and come as scalar operands, half a row ahead; from LDS they took longer than the
+// vector work at M_4.  Small grids share out the ordinates over the blocks.
+// *wild is set where a value is not a number or exceeds kTame (see k_stencil).
+constexpr double kTame = 1e290;
+template <int NM>
+__global__ __launch_bounds__(kTB) void k_ansatz(int64_t ng, int nq, int nqPer,
+                                                 const double *__restrict__ ord,
+                                                 const double *__restrict__ alpha, double *A,
+                                                 int isPn, int *wild)
+{
+    constexpr int HA = (NM + 1) / 2, HB = NM - HA;
     const int64_t cell = (int64_t)blockIdx.x * kTB + threadIdx.x;
     const bool have = cell < ng;
     double a[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m)
         a[m] = have ? alpha[cell * NM + m] : 0.0;
-    for (int q0 = 0; q0 < nq; q0 += kChunk) {
-        const int nqc = min(kChunk, nq - q0);
-        __syncthreads();
-        for (int e = threadIdx.x; e < nqc * NM; e += kTB)
-            sM[e] = M[(size_t)q0 * NM + e];
-        __syncthreads();
-        if (have) {
-            for (int ql = 0; ql < nqc; ++ql) {
-                double kin = 0.0;
+    const int q0 = blockIdx.y * nqPer, q1 = min(q0 + nqPer, nq);
+    if (q0 >= q1)
+        return;
+    const double *row = ord + (size_t)q0 * ord_row(NM) + 4;
+    double *At = A + (size_t)q0 * ng + cell;
+    double mA[HA];
+    bool bad = false;
 #pragma unroll
-                for (int m = 0; m < NM; ++m)
-                    kin += a[m] * sM[ql * NM + m];
-                A[(size_t)(q0 + ql) * ng + cell] =
-                    isPn == 1 ? kin : (isPn == 2 ? det_exp(kin) : exp(kin));
-            }
-        }
+    for (int m = 0; m < HA; ++m)
+        mA[m] = row[m];
+#pragma unroll 1
+    for (int q = q0; q < q1; ++q) {
+        double mB[HB], kin = 0.0;
+        __builtin_amdgcn_sched_barrier(0);
+        use_s(mA);
+#pragma unroll
+        for (int m = 0; m < HB; ++m)
+            mB[m] = row[HA + m];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < HA; ++m)
+            kin += a[m] * mA[m];
+        __builtin_amdgcn_sched_barrier(0);
+        use_s(mB);
+        row += ord_row(NM);  // past the last row: padding
+#pragma unroll
+        for (int m = 0; m < HA; ++m)
+            mA[m] = row[m];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < HB; ++m)
+            kin += a[HA + m] * mB[m];
+        const double v = isPn == 1 ? kin : (isPn == 2 ? det_exp(kin) : exp(kin));
+        bad |= !(fabs(v) <= kTame);
+        if (have)
+            *At = v;
+        At += ng;
     }
+    if (have && bad)
+        *wild = 1;
 }
+__global__ void k_clear_int(int *p) { *p = 0; }
 
 __device__ __forceinline__ double sgn1(double x) { return x >= 0.0 ? 1.0 : -1.0; }
 __device__ __forceinline__ double mmin(double a, double b) { return a < b ? a : b; }
@@ -207,7 +251,8 @@ struct StencilArgs {
     int nq;
     double dx, dy, dz, theta, dt;
     int fuseEuler;
-    double rdx, rdy, rdz;  // 1/dx, ... (used when every spacing is a power of two)
+    double rdx, rdy, rdz;  // 1/dx, ...
+    int general;           // take the general path whatever the ansatz holds
 };
 
 // x / d == x * (1/d) exactly, for every x, iff d is a power of two
@@ -217,66 +262,226 @@ bool exact_reciprocal(double d)
     return d > 0.0 && std::isfinite(d) && std::frexp(d, &e) == 0.5 && e > -1021 && e < 1022;
 }
 
-// P2: dx, dy, dz powers of two (division by them is multiplication by exact reciprocals)
-template <int NM, bool P2, bool TH1>
+typedef const __attribute__((address_space(1))) double GlobalDouble;
+typedef const __attribute__((address_space(1))) char GlobalByte;
+
+// The three-way minmod that slopefit's nested one is for ordinary numbers (the common sign's
+// smallest magnitude, else 0): y limited to what x and z of one sign leave of [n, p].
+__device__ __forceinline__ double minmod3(double x, double y, double z)
+{
+    const double p = fmax(0.0, fmin(x, z)), n = fmin(0.0, fmax(x, z));
+    return fmax(n, fmin(p, y));
+}
+// axis_flux on the four values it reads: u2, u1 upwind of the centre, a0, and d1 downwind.
+// For dir <= 0 the axis is mirrored, which negates both slopes exactly.  The halves are
+// moved through the minima (a factor of two commutes with every operation) to where one
+// fused multiply-add, whose product is exact, adds the limited half slope.  th2 = 2 theta.
+template <bool TH1>
+__device__ __forceinline__ double upwind_flux(double u2, double u1, double a0, double d1,
+                                              double dir, bool pos, double wq, double th2)
+{
+    double zA = u1 - u2, zB = a0 - u1, zC = d1 - a0, yA = a0 - u2, yB = d1 - u1;
+    if constexpr (TH1) {
+        yA = 0.5 * yA;
+        yB = 0.5 * yB;
+    } else {
+        zA = th2 * zA;
+        zB = th2 * zB;
+        zC = th2 * zC;
+    }
+    constexpr double h = TH1 ? 0.5 : 0.25;
+    const double sA = minmod3(zB, yA, zA), sB = minmod3(zC, yB, zB);
+    double f;
+    if (pos)
+        f = fma(-h, sA, fma(h, sB, a0) - u1);
+    else
+        f = fma(-h, sB, fma(h, sA, u1) - a0);
+    return f * dir * wq;
+}
+// x / d from the correctly rounded r = 1 / d: one residual correction gives the correctly
+// rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990) away from the ends of the
+// exponent range; three operations instead of the dozen of a division.
+__device__ __forceinline__ double div_by(double x, double d, double r)
+{
+    const double q = x * r;
+    return fma(fma(-q, d, x), r, q);
+}
+
+// sum_q m_q (Fx/dx + Fy/dy + Fz/dz) for one interior cell per thread, optionally with the Euler
+// stage.  Bound by the vector unit: at theta != 1 and general spacings about 105 operations for
+// the three axes and 2 NM for the moments, per cell and ordinate.  What keeps it there:
+//   - upwind_flux: the limiter as minima and maxima, four values an axis, the differences of
+//     its two slopes shared (the nested minmod with its sign products took twice as many);
+//   - div_by instead of division (or, P2: every spacing a power of two, the exact reciprocal);
+//   - D ordinates' values in flight per thread: 2 where waves enough hide the latency, 4 on
+//     grids that leave the chip mostly idle;
+//   - the ordinate table as scalar operands, issued a stage ahead;
+//   - the tiling above, for the L2.
+// All of it gives the general path's bits as long as the ansatz is at most kTame, spacings and
+// theta are within reason and (Markstein) no axis's flux is below 1e-290; a NaN or a larger
+// value anywhere (*wild, from k_ansatz) sends the whole call down the general path.
+// Measured, ansatz and stencil together, against a kernel with 13 loads, the nested limiter and
+// divisions: M_3 Q = 12 61x45x77 theta = 2: 945 -> 760 us; 96x128x128: 5.80 -> 4.60 ms; 16x12x20:
+// 535 -> 220 us; M_2 20^3 step, flux share: 220 -> 80 us.  The vector unit is busy 56% of the
+// large grid's time (855 M instructions); the L1 serves 10 unaligned rows per cell and ordinate.
+template <int NM, bool P2, bool TH1, int D>
 __global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__restrict__ A,
-                                                  const double *__restrict__ M,
-                                                  const double *__restrict__ xi,
-                                                  const double *__restrict__ eta,
-                                                  const double *__restrict__ mu,
-                                                  const double *__restrict__ w, double *flux,
+                                                  const double *__restrict__ ord,
+                                                  const int *__restrict__ sgn,
+                                                  const int *__restrict__ wild, double *flux,
                                                   double *u, const double *__restrict__ sigT,
                                                   const double *__restrict__ sigS)
 {
+    constexpr int OR = ord_row(NM);
     const Grid &G = S.G;
-    const int64_t ni = (int64_t)G.nx * G.ny * G.nz;
-    const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
-    if (t >= ni)
+    Tile T;
+    if (!tile_of(G, T))
         return;
-    const int k = 2 + (int)(t % G.nz);
-    const int j = 2 + (int)((t / G.nz) % G.ny);
-    const int i = 2 + (int)(t / ((int64_t)G.nz * G.ny));
+    const int64_t np = (int64_t)G.ny * G.nz;
+    const int64_t p = T.p + threadIdx.x;
+    const bool have = p < np;
+    // lanes past the plane's end work on its last cell and write nothing
+    const int64_t pc = have ? p : np - 1;
+    const int j = 2 + (int)(pc / G.nz), k = 2 + (int)(pc % G.nz);
     const size_t ng = (size_t)G.NX * G.NY * G.NZ;
-    const size_t c = G.idx(i, j, k);
-    const size_t sx = (size_t)G.NY * G.NZ, sy = (size_t)G.NZ;
+    const size_t c = G.idx(T.i, j, k);
+    const ptrdiff_t sx = (ptrdiff_t)G.NY * G.NZ, sy = G.NZ;
     double fl[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m)
         fl[m] = 0.0;
-    // the 13 ansatz values of the cell's stencil at ordinate q: the centre, then -2, -1, +1,
-    // +2 along x, y and z; the next ordinate's are in flight while this one's are used
-    const ptrdiff_t off[13] = {0,
-                               -2 * (ptrdiff_t)sx, -(ptrdiff_t)sx, (ptrdiff_t)sx, 2 * (ptrdiff_t)sx,
-                               -2 * (ptrdiff_t)sy, -(ptrdiff_t)sy, (ptrdiff_t)sy, 2 * (ptrdiff_t)sy,
-                               -2, -1, 1, 2};
-    double v[13], nv[13];
+    if (!S.general && *wild == 0) {
+        const unsigned inPlane = 8u * ((unsigned)j * (unsigned)G.NZ + (unsigned)k);
+        const double *plane = A + (size_t)T.i * sx;
+        // the values of the ordinate at plane b whose direction signs are sg (bits x, y, z; set:
+        // positive)
+        auto load = [&](double(&v)[10], const double *b, int sg) {
+            unsigned off = inPlane;
+            asm("" : "+v"(off));  // widened here, next to the loads
+            auto at = [&](ptrdiff_t o) {
+                // the base stays scalar: one register offset serves every load
+                uint64_t base = (uint64_t)(b + o);
+                asm("" : "+s"(base));
+                return *(GlobalDouble *)((GlobalByte *)base + off);
+            };
+            v[0] = at(0);
 #pragma unroll
-    for (int e = 0; e < 13; ++e)
-        v[e] = A[c + off[e]];
-    for (int q = 0; q < S.nq; ++q) {
-        if (q + 1 < S.nq) {
-            const double *An = A + (size_t)(q + 1) * ng + c;
+            for (int ax = 0; ax < 3; ++ax) {
+                const ptrdiff_t st = ax == 0 ? sx : (ax == 1 ? sy : 1);
+                const ptrdiff_t up = (sg >> ax) & 1 ? -st : st;
+                v[1 + 3 * ax] = at(2 * up);
+                v[2 + 3 * ax] = at(up);
+                v[3 + 3 * ax] = at(-up);
+            }
+        };
+        double v[D][10], dirs[4];
+        int sNow[D], sNext;  // signs of the ordinates in v; of the one loaded next
 #pragma unroll
-            for (int e = 0; e < 13; ++e)
-                nv[e] = An[off[e]];
+        for (int d = 0; d < D; ++d) {
+            sNow[d] = sgn[d];
+            load(v[d], plane, sNow[d]);
+            plane += d + 1 < S.nq ? ng : 0;
+            __builtin_amdgcn_sched_barrier(0);  // in order, as the counted waits need them
         }
-        const double a0 = v[0];
-        const double wq = w[q];
-        const double fX = axis_flux<TH1>(v[1], v[2], a0, v[3], v[4], xi[q], wq, S.theta);
-        const double fY = axis_flux<TH1>(v[5], v[6], a0, v[7], v[8], eta[q], wq, S.theta);
-        const double fZ = axis_flux<TH1>(v[9], v[10], a0, v[11], v[12], mu[q], wq, S.theta);
+        sNext = sgn[D];
 #pragma unroll
-        for (int e = 0; e < 13; ++e)
-            v[e] = nv[e];
-        double s;
-        if constexpr (P2)
-            s = fX * S.rdx + fY * S.rdy + fZ * S.rdz;
-        else
-            s = fX / S.dx + fY / S.dy + fZ / S.dz;
+        for (int e = 0; e < 4; ++e)
+            dirs[e] = ord[e];
+        const double *row = ord;
+        // the scalar registers are for the ordinate table: the constants go to vector ones
+        double th2 = 2.0 * S.theta, hx = S.dx, hy = S.dy, hz = S.dz, rx = S.rdx, ry = S.rdy,
+               rz = S.rdz;
+        asm("" : "+v"(th2), "+v"(hx), "+v"(hy), "+v"(hz), "+v"(rx), "+v"(ry), "+v"(rz));
+        auto ordinate = [&](int d, int q) {
+            // M's row in pieces of at most nine, for the scalar registers; a piece is issued
+            // before the one ahead of it is used
+            constexpr int PS = NM <= 9 ? NM : (NM == 16 ? 8 : 9), NP = (NM + PS - 1) / PS;
+            double m[2][PS];
+            auto piece = [&](int p) {
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-            fl[m] += M[(size_t)q * NM + m] * s;
+                for (int i = 0; i < PS; ++i)
+                    m[p & 1][i] = p * PS + i < NM ? row[4 + p * PS + i] : 0.0;
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            use_s(dirs);
+            asm volatile("" ::"s"(sNext));
+            piece(0);
+            __builtin_amdgcn_sched_barrier(0);
+            const int sg = sNow[d];
+            const double(&w)[10] = v[d];
+            const double wq = dirs[3];
+            const double fX = upwind_flux<TH1>(w[1], w[2], w[0], w[3], dirs[0], sg & 1, wq, th2);
+            const double fY = upwind_flux<TH1>(w[4], w[5], w[0], w[6], dirs[1], sg & 2, wq, th2);
+            const double fZ = upwind_flux<TH1>(w[7], w[8], w[0], w[9], dirs[2], sg & 4, wq, th2);
+            double s;
+            if constexpr (P2)
+                s = fX * rx + fY * ry + fZ * rz;
+            else
+                s = div_by(fX, hx, rx) + div_by(fY, hy, ry) + div_by(fZ, hz, rz);
+            __builtin_amdgcn_sched_barrier(0);
+            sNow[d] = sNext;
+            // unconditional (at the end again the last plane), so that the waits for the values
+            // in flight can be counted
+            load(v[d], plane, sNow[d]);
+            plane += q + D + 1 < S.nq ? ng : 0;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                use_s(m[p & 1]);
+                if (p + 1 < NP) {
+                    piece(p + 1);
+                } else {
+                    row += OR;  // past the last row: padding
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        dirs[e] = row[e];
+                    sNext = sgn[q + 1 + D];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < PS && p * PS + i < NM; ++i)
+                    fl[p * PS + i] += m[p & 1][i] * s;
+                if (p + 1 < NP)
+                    __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int q0 = 0;
+#pragma unroll 1
+        for (; q0 + D <= S.nq; q0 += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+                ordinate(d, q0 + d);
+        }
+        if constexpr (D > 2) {  // nq is even
+#pragma unroll 1
+            for (int d = 0; q0 + d < S.nq; ++d) {
+                ordinate(0, q0 + d);
+#pragma unroll
+                for (int e = 0; e < 10; ++e)
+                    v[0][e] = v[1][e];
+                sNow[0] = sNow[1];
+            }
+        }
+    } else {
+        for (int q = 0; q < S.nq; ++q) {
+            const double *a = A + (size_t)q * ng + c, *row = ord + (size_t)q * OR;
+            const double a0 = a[0], wq = row[3];
+            const double fX = axis_flux<TH1>(a[-2 * sx], a[-sx], a0, a[sx], a[2 * sx], row[0],
+                                             wq, S.theta);
+            const double fY = axis_flux<TH1>(a[-2 * sy], a[-sy], a0, a[sy], a[2 * sy], row[1],
+                                             wq, S.theta);
+            const double fZ = axis_flux<TH1>(a[-2], a[-1], a0, a[1], a[2], row[2], wq, S.theta);
+            double s;
+            if constexpr (P2)
+                s = fX * S.rdx + fY * S.rdy + fZ * S.rdz;
+            else
+                s = fX / S.dx + fY / S.dy + fZ / S.dz;
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+                fl[m] += row[4 + m] * s;
+        }
     }
+    if (!have)
+        return;
     if (S.fuseEuler) {
         // update.cpp:28-35
         const double dt = S.dt, st = sigT[c], ss = sigS[c];
@@ -692,15 +897,25 @@ hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *a
     if (!isPn && ctx->precision == C3D_PREC_FP64_REFORDER)
         isPn = 2;
     const int64_t ng = (int64_t)(nx + 4) * (ny + 4) * (nz + 4);
-    dim3 grid(blocks_for(ng, kTB, INT32_MAX));
     const int nq = ctx->t.nq;
+    // small grids share out the ordinates too: 8 blocks a CU, at least 16 ordinates each
+    const int64_t bx = blocks_for(ng, kTB, INT32_MAX);
+    const int64_t want = std::max<int64_t>(1, (int64_t)ctx->numCU * 8 / bx);
+    const int split = (int)std::min<int64_t>(want, (nq + 15) / 16);
+    const int nqPer = (nq + split - 1) / split;
+    dim3 grid((unsigned)bx, (unsigned)split);
+    hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, ctx->d_wild);
+#define C3D_ANSATZ(NMV)                                                                        \
+    hipLaunchKernelGGL(k_ansatz<NMV>, grid, dim3(kTB), 0, s, ng, nq, nqPer, ctx->d_ord, \
+                       alpha, A, isPn, ctx->d_wild)
     switch (ctx->t.nm) {
-    case 4: hipLaunchKernelGGL(k_ansatz<4>, grid, dim3(kTB), 0, s, ng, nq, ctx->d_M, alpha, A, isPn); break;
-    case 9: hipLaunchKernelGGL(k_ansatz<9>, grid, dim3(kTB), 0, s, ng, nq, ctx->d_M, alpha, A, isPn); break;
-    case 16: hipLaunchKernelGGL(k_ansatz<16>, grid, dim3(kTB), 0, s, ng, nq, ctx->d_M, alpha, A, isPn); break;
-    case 25: hipLaunchKernelGGL(k_ansatz<25>, grid, dim3(kTB), 0, s, ng, nq, ctx->d_M, alpha, A, isPn); break;
+    case 4: C3D_ANSATZ(4); break;
+    case 9: C3D_ANSATZ(9); break;
+    case 16: C3D_ANSATZ(16); break;
+    case 25: C3D_ANSATZ(25); break;
     default: return hipErrorInvalidValue;
     }
+#undef C3D_ANSATZ
     return hipGetLastError();
 }
 
@@ -709,29 +924,40 @@ hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *
                           double dx, double dy, double dz, double theta, int fuseEuler,
                           int zeroGhosts, hipStream_t s)
 {
+    auto tame = [](double x) { return fabs(x) > 1e-15 && fabs(x) < 1e15; };
     StencilArgs S{make_grid(nx, ny, nz), ctx->t.nq, dx, dy, dz, theta, dt, fuseEuler,
-                  1.0 / dx, 1.0 / dy, 1.0 / dz};
+                  1.0 / dx, 1.0 / dy, 1.0 / dz, 0};
+    // a plane's offsets are 32 bits of bytes on the fast path
+    S.general = !(tame(dx) && tame(dy) && tame(dz) && fabs(theta) < 1e15 &&
+                  (int64_t)S.G.NY * S.G.NZ < (1 << 29));
     const bool p2 = exact_reciprocal(dx) && exact_reciprocal(dy) && exact_reciprocal(dz);
     const bool th1 = theta == 1.0;
-    const int64_t ni = (int64_t)nx * ny * nz;
-    dim3 grid(blocks_for(ni, kTB, INT32_MAX));
+    dim3 grid(tile_blocks(S.G));
+    // four ordinates in flight where there is at most a wave per SIMD
+    const bool deep = grid.x <= (unsigned)ctx->numCU;
     if (zeroGhosts && !fuseEuler) {
         const int64_t ng = (int64_t)S.G.NX * S.G.NY * S.G.NZ;
         hipLaunchKernelGGL(k_zero_ghost_flux, dim3(blocks_for(ng * ctx->t.nm, 256, 65536)),
                            dim3(256), 0, s, S.G, ctx->t.nm, flux);
     }
-#define C3D_STENCIL_V(NMV, P, T)                                                              \
-    hipLaunchKernelGGL((k_stencil<NMV, P, T>), grid, dim3(kTB), 0, s, S, A, ctx->d_M,          \
-                       ctx->d_xi, ctx->d_eta, ctx->d_mu, ctx->d_w, flux, u, sigmaT, sigmaS)
-#define C3D_STENCIL(NMV)                                                                      \
+#define C3D_STENCIL_V(NMV, P, T, D)                                                           \
+    hipLaunchKernelGGL((k_stencil<NMV, P, T, D>), grid, dim3(kTB), 0, s, S, A, ctx->d_ord,     \
+                       ctx->d_sgn, ctx->d_wild, flux, u, sigmaT, sigmaS)
+#define C3D_STENCIL_D(NMV, D)                                                                 \
     if (p2 && th1)                                                                             \
-        C3D_STENCIL_V(NMV, true, true);                                                        \
+        C3D_STENCIL_V(NMV, true, true, D);                                                     \
     else if (p2)                                                                               \
-        C3D_STENCIL_V(NMV, true, false);                                                       \
+        C3D_STENCIL_V(NMV, true, false, D);                                                    \
     else if (th1)                                                                              \
-        C3D_STENCIL_V(NMV, false, true);                                                       \
+        C3D_STENCIL_V(NMV, false, true, D);                                                    \
     else                                                                                       \
-        C3D_STENCIL_V(NMV, false, false)
+        C3D_STENCIL_V(NMV, false, false, D)
+#define C3D_STENCIL(NMV)                                                                      \
+    if (deep) {                                                                                \
+        C3D_STENCIL_D(NMV, 4);                                                                 \
+    } else {                                                                                   \
+        C3D_STENCIL_D(NMV, 2);                                                                 \
+    }
     switch (ctx->t.nm) {
     case 4: C3D_STENCIL(4); break;
     case 9: C3D_STENCIL(9); break;
@@ -740,6 +966,7 @@ hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *
     default: return hipErrorInvalidValue;
     }
 #undef C3D_STENCIL
+#undef C3D_STENCIL_D
 #undef C3D_STENCIL_V
     return hipGetLastError();
 }
