@@ -155,28 +155,58 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ double wave_sum(double v)
+// v of the partner lane at distance 8, 4, 2, 1 (lane ^ O) within the 16-lane row, on the vector
+// unit.  Taken in that order by a butterfly: the rotation by 4 reaches lane ^ 4 or lane ^ 12,
+// which hold the same value once the partners at distance 8 are combined.
+template <int O>
+__device__ __forceinline__ int row_partner(int v)
 {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1)
-        v = v + __shfl_xor(v, o);
-    return v;
+    constexpr int ctrl = O == 8 ? 0x128 : (O == 4 ? 0x124 : (O == 2 ? 0x4E : 0xB1));
+    return __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, false);
+}
+template <int O>
+__device__ __forceinline__ double row_partner(double v)
+{
+    return __hiloint2double(row_partner<O>(__double2hiint(v)),
+                            row_partner<O>(__double2loint(v)));
+}
+template <int O>
+__device__ __forceinline__ float row_partner(float v)
+{
+    return __int_as_float(row_partner<O>(__float_as_int(v)));
+}
+// v + v of lane ^ 32 (lane ^ 16): the swaps give every lane both halves' (rows') values
+__device__ __forceinline__ double half_sum(double v)
+{
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const u2 l = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const u2 h = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+__device__ __forceinline__ double rows_sum(double v)
+{
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const u2 l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const u2 h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
 }
 
 // Sum over the lane's 16-lane row (butterfly: every lane of the row gets the same bits).
 __device__ __forceinline__ double row16_sum(double v)
 {
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1)
-        v = v + __shfl_xor(v, o);
-    return v;
+    v = v + row_partner<8>(v);
+    v = v + row_partner<4>(v);
+    v = v + row_partner<2>(v);
+    return v + row_partner<1>(v);
 }
+// ... over the wave, partners at distance 32, 16, 8, ..., 1
+__device__ __forceinline__ double wave_sum(double v) { return row16_sum(rows_sum(half_sum(v))); }
 __device__ __forceinline__ float row16_max(float v)
 {
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1)
-        v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    v = fmaxf(v, row_partner<8>(v));
+    v = fmaxf(v, row_partner<4>(v));
+    v = fmaxf(v, row_partner<2>(v));
+    return fmaxf(v, row_partner<1>(v));
 }
 
 // A cell's lanes: the whole wave (G = 64, one cell per wave; broadcasts by readlane), one
@@ -3482,89 +3512,106 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
 }
 
-// f alone for one cell at kw <= KW trial points (one wave; the points in LDS, KW x NM), for
+// f alone for one cell at KW trial points (one wave; the points in LDS, KW x NM), for
 // line-search trials in the tail kernel: sum_q w_q exp(alpha.m_q) with exactly the
 // operations the sweep kernels use for that sum, so that a cell's result does not depend on
 // which kernel evaluated it -- kFp64: chunk_mfma's exponent, per-lane partials over the
 // chunks and final wave_sum; kFRef: chunk_ref's deterministic exp and ordinate-order sum
 // (one point).  (The mixed phase's points: f_trials_mixed.)  M is read from the transposed
-// table MT [NM][nqPad] (one coalesced load per component), two chunks in flight, each chunk's
-// M shared by the kw points.
+// table MT [NM][nqPad] (one coalesced load per component), each chunk's M shared by the points.
+// Bound by latency: the wave is alone on its SIMD, so all points' exponents and exps run side
+// by side, with few points those of two chunks (their terms are added in chunk order), and the
+// next chunks are in flight meanwhile; the point count is a constant, since a test per point
+// would end each chain before the next starts.
 enum : int { kFp64 = 0, kFRef = 1 };
 template <int NM, int MODE, int KW>
 __device__ __forceinline__ void f_trials(const KParams &P, const double *__restrict__ MT,
                                          const double *__restrict__ wg, const double *sA,
-                                         int kw, double *sW, double *sE, int lane,
-                                         double (&out)[KW])
+                                         double *sW, double *sE, int lane, double (&out)[KW])
 {
     static_assert(MODE != kFRef || KW == 1, "reference order: one point per wave");
     const int nch = P.nqPad / kChunk;
     const size_t ld = (size_t)P.nqPad;
-    double mA[NM], mB[NM], wA = 0.0, wB = 0.0;
-    // kFp64 evaluates ordinate mfma_ordinate(lane) of each chunk, as chunk_mfma does
-    const int qo = MODE == kFp64 ? mfma_ordinate(lane) : lane;
-    auto load = [&](double(&m)[NM], double &w, int ch) {
-        const size_t q = (size_t)ch * kChunk + qo;
-#pragma unroll
-        for (int i = 0; i < NM; ++i)
-            m[i] = MT[i * ld + q];
-        w = wg[q];
-    };
     double fpart[KW];
 #pragma unroll
     for (int j = 0; j < KW; ++j)
         fpart[j] = 0.0;
-    auto term = [&](const double(&m)[NM], double w, int ch) {
-#pragma unroll
-        for (int j = 0; j < KW; ++j) {
-            if (j >= kw)
-                continue;
-            const double *a = sA + j * NM;
+    if constexpr (MODE == kFRef) {
+        for (int ch = 0; ch < nch; ++ch) {
+            const size_t q = (size_t)ch * kChunk + lane;
             double x = 0.0;
-            {
-                if constexpr (MODE == kFRef) {
+#pragma unroll
+            for (int i = 0; i < NM; ++i)
+                x = x + sA[i] * MT[i * ld + q];
+            wave_lds_sync();
+            sE[lane] = det_exp(x);
+            sW[lane] = wg[q];
+            wave_lds_sync();
+            const int nqc = min(kChunk, P.nq - ch * kChunk);
+            for (int k = 0; k < nqc; ++k)
+                fpart[0] = fpart[0] + sW[k] * sE[k];
+        }
+        out[0] = fpart[0];
+    } else {
+        // ordinate mfma_ordinate(lane) of each chunk, as chunk_mfma does; a chunk past the last
+        // is the last one again, left out of the sum
+        constexpr int H = KW >= 4 ? 1 : 2;  // chunks side by side
+        constexpr int NB = KW >= 4 ? 2 : 1;  // and such groups in flight
+        struct Group {
+            double m[H][NM], w[H];
+        };
+        const double *Mq = MT + mfma_ordinate(lane), *wq = wg + mfma_ordinate(lane);
+        auto load = [&](Group &b, int ch) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const size_t q = (size_t)min(ch + h, nch - 1) * kChunk;
+#pragma unroll
+                for (int i = 0; i < NM; ++i)
+                    b.m[h][i] = Mq[i * ld + q];
+                b.w[h] = wq[q];
+            }
+        };
+        auto term = [&](Group &b, int ch) {
+            double e[H][KW], w[H];
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+#pragma unroll
+                for (int j = 0; j < KW; ++j) {
+                    double x = 0.0;
 #pragma unroll
                     for (int i = 0; i < NM; ++i)
-                        x = x + a[i] * m[i];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < NM; ++i)
-                        x = fma(a[i], m[i], x);
+                        x = fma(sA[j * NM + i], b.m[h][i], x);
+                    e[h][j] = x;
                 }
-                if constexpr (MODE == kFRef) {
-                    wave_lds_sync();
-                    sE[lane] = det_exp(x);
-                    sW[lane] = w;
-                    wave_lds_sync();
-                    const int nqc = min(kChunk, P.nq - ch * kChunk);
-                    for (int k = 0; k < nqc; ++k)
-                        fpart[j] = fpart[j] + sW[k] * sE[k];
-                } else {
-                    fpart[j] = fpart[j] + w * exp(x);
+                w[h] = b.w[h];
+            }
+            load(b, ch + H * NB);
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+#pragma unroll
+                for (int j = 0; j < KW; ++j)
+                    e[h][j] = w[h] * exp(e[h][j]);
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const bool in = ch + h < nch;
+#pragma unroll
+                for (int j = 0; j < KW; ++j) {
+                    const double f2 = fpart[j] + e[h][j];
+                    fpart[j] = in ? f2 : fpart[j];
                 }
             }
-        }
-    };
-    load(mA, wA, 0);
-    if (nch > 1)
-        load(mB, wB, 1);
-    for (int ch = 0; ch < nch; ch += 2) {
-        term(mA, wA, ch);
-        if (ch + 2 < nch)
-            load(mA, wA, ch + 2);
-        if (ch + 1 < nch) {
-            term(mB, wB, ch + 1);
-            if (ch + 3 < nch)
-                load(mB, wB, ch + 3);
-        }
-    }
+        };
+        Group b[NB];
 #pragma unroll
-    for (int j = 0; j < KW; ++j) {
-        if (j >= kw)
-            continue;
-        if constexpr (MODE == kFRef)
-            out[j] = fpart[j];
-        else
+        for (int p = 0; p < NB; ++p)
+            load(b[p], H * p);
+#pragma unroll 1
+        for (int ch = 0; ch < nch; ch += H * NB)
+#pragma unroll
+            for (int p = 0; p < NB; ++p)
+                term(b[p], ch + H * p);
+#pragma unroll
+        for (int j = 0; j < KW; ++j)
             out[j] = wave_sum(fpart[j]);
     }
 }
@@ -3680,7 +3727,7 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
     constexpr int NMS = NM | 1;
     // trial points per wave in a wide round: as many as keep a round's latency near one f
     // evaluation's (f costs nq (NM + exp) per point)
-    constexpr int KW = REF ? 1 : (NM <= 9 ? 8 : (NM <= 16 ? 2 : 1));
+    constexpr int KW = REF ? 1 : (NM <= 9 ? 8 : (NM <= 16 ? 4 : 1));
     // in the mixed phase the points are the rows of the exponent products: four per wave
     constexpr int KWM = 4;
     constexpr int KWA = MIXED && KWM > KW ? KWM : KW;
@@ -3737,9 +3784,7 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                 // mixed phase's points are the rows of one exponent product, so its four cost
                 // what one does and are taken from the first trial on
                 const int kw = mx ? KWM : (C.tls < 1.0 ? KW : 1);
-                double tk = C.tls;
-                for (int k = 0; k < wv * kw; ++k)
-                    tk = 0.5 * tk;
+                double tk = ldexp(C.tls, -wv * kw);
                 auto point = [&](int j, double t) {
                     return (wv == 0 && j == 0) ? C.a : (li < NM ? C.aOld + t * C.d : 0.0);
                 };
@@ -3762,9 +3807,17 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                         for (int j = 0; j < KWA; ++j)
                             ft[j] = j < 4 ? f4p[j] : 0.0;
                     } else {
+                        constexpr int MODE = REF ? kFRef : kFp64;
                         double fk[KW];
-                        f_trials<NM, REF ? kFRef : kFp64, KW>(P, MT, wg, sA[wv], kw, sW[wv],
-                                                              sE[wv], lane, fk);
+                        if (KW > 1 && kw == 1) {
+                            double f1[1];
+                            f_trials<NM, MODE, 1>(P, MT, wg, sA[wv], sW[wv], sE[wv], lane, f1);
+#pragma unroll
+                            for (int j = 0; j < KW; ++j)
+                                fk[j] = j == 0 ? f1[0] : 0.0;
+                        } else {
+                            f_trials<NM, MODE, KW>(P, MT, wg, sA[wv], sW[wv], sE[wv], lane, fk);
+                        }
 #pragma unroll
                         for (int j = 0; j < KWA; ++j)
                             ft[j] = j < KW ? fk[j] : 0.0;
@@ -3781,15 +3834,20 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                     }
                 }
                 __syncthreads();
-                bool accepted = false;
-                for (int k = 0; k < TW * kw; ++k) {
-                    if (sOk[k]) {
-                        accepted = true;
-                        break;
-                    }
-                    C.ls_reject(li);  // halve the step, or give up
-                    if (C.phase != kPhaseLS)
-                        break;
+                // The search over the verdicts in order: at trial k it accepts, or halves the
+                // step (ls_reject) and gives up if that is too short.  Lane k looks at trial k.
+                const int n = TW * kw;
+                static_assert(TW * KWA <= kWave, "a lane per trial");
+                const bool okK = lane < n && sOk[lane < n ? lane : 0];
+                const bool deadK =
+                    lane < n && !(ldexp(C.tls, -(lane + 1)) * C.maxF > DBL_EPSILON / 2);
+                const unsigned long long okM = __ballot(okK), deadM = __ballot(deadK);
+                const int kOk = okM ? __ffsll(okM) - 1 : n, kDead = deadM ? __ffsll(deadM) - 1 : n;
+                const bool accepted = kOk < n && kOk <= kDead;
+                if (accepted ? kOk > 0 : n > 0) {  // the last rejection, with its ls_next()
+                    const int last = accepted ? kOk : min(kDead + 1, n);
+                    C.tls = ldexp(C.tls, 1 - last);
+                    C.ls_reject(li);
                 }
                 __syncthreads();  // sOk and sA are rewritten by the next round
                 if (!accepted)
