@@ -3730,8 +3730,11 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
     constexpr int NB = NT * (NT + 1) / 2;
     constexpr int NMS = NM | 1;
     // trial points per wave in a wide round: as many as keep a round's latency near one f
-    // evaluation's (f costs nq (NM + exp) per point)
-    constexpr int KW = REF ? 1 : (NM <= 9 ? 8 : (NM <= 16 ? 4 : 1));
+    // evaluation's (f costs nq (NM + exp) per point) and the registers allow
+    constexpr int KW = REF ? 1 : (NM <= 9 ? 8 : (NM <= 16 ? (MIXED ? 2 : 4) : 1));
+    // points side by side: the mixed kernel at nm = 9 would spill with eight (M_2 closure of 3000
+    // cells 2.87 -> 3.17 ms)
+    constexpr int KB = MIXED && NM == 9 ? 4 : KW;
     // in the mixed phase the points are the rows of the exponent products: four per wave
     constexpr int KWM = 4;
     constexpr int KWA = MIXED && KWM > KW ? KWM : KW;
@@ -3820,7 +3823,15 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                             for (int j = 0; j < KW; ++j)
                                 fk[j] = j == 0 ? f1[0] : 0.0;
                         } else {
-                            f_trials<NM, MODE, KW>(P, MT, wg, sA[wv], sW[wv], sE[wv], lane, fk);
+#pragma unroll
+                            for (int j0 = 0; j0 < KW; j0 += KB) {
+                                double fb[KB];
+                                f_trials<NM, MODE, KB>(P, MT, wg, sA[wv] + j0 * NM, sW[wv],
+                                                       sE[wv], lane, fb);
+#pragma unroll
+                                for (int j = 0; j < KB; ++j)
+                                    fk[j0 + j] = fb[j];
+                            }
                         }
 #pragma unroll
                         for (int j = 0; j < KWA; ++j)
