@@ -3734,7 +3734,7 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
     constexpr int KW = REF ? 1 : (NM <= 9 ? 8 : (NM <= 16 ? (MIXED ? 2 : 4) : 1));
     // points side by side: the mixed kernel at nm = 9 would spill with eight (M_2 closure of 3000
     // cells 2.87 -> 3.17 ms)
-    constexpr int KB = MIXED && NM == 9 ? 4 : KW;
+    constexpr int KB = MIXED && NM <= 9 ? 4 : KW;
     // in the mixed phase the points are the rows of the exponent products: four per wave
     constexpr int KWM = 4;
     constexpr int KWA = MIXED && KWM > KW ? KWM : KW;
