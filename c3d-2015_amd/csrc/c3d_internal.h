@@ -97,7 +97,8 @@ struct c3d_ctx_s {
     double *d_w = nullptr, *d_xi = nullptr, *d_eta = nullptr, *d_mu = nullptr;
     double *d_ord = nullptr;   // [nq + 2][4 + nm], rows (xi, eta, mu, w, M's row); two zero rows
     int32_t *d_sgn = nullptr;  // [nq + 8], bits 0..2: xi, eta, mu > 0
-    int *d_wild = nullptr;     // the ansatz holds a NaN or a huge value (grid.hip)
+    int *d_wild = nullptr;     // the ansatz holds a NaN, a huge or a tiny value (grid.hip)
+    bool tameOrdinates = false;  // directions and weights of ordinary size (grid.hip)
     double *d_M = nullptr;     // [nqPad][nm], rows >= nq zero
     double *d_MT = nullptr;    // [nm][nqPad], the transpose of d_M
     double *d_wpad = nullptr;  // [nqPad], entries >= nq zero
@@ -179,7 +180,7 @@ int mlp_get(c3d_ctx_s *ctx, float *params, float *norm);
 hipError_t launch_ghost_fill(int nx, int ny, int nz, int nm, double *u, hipStream_t s,
                              double *u2 = nullptr);
 hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *alpha,
-                         double *A, int isPn, hipStream_t s);
+                         double *A, int isPn, double dx, double dy, double dz, hipStream_t s);
 hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *A,
                           double *flux, double *u, const double *sigmaT,
                           const double *sigmaS, double dt, double dx, double dy, double dz,

@@ -101,7 +101,11 @@ int finish_ctx(c3d_ctx_s *ctx)
         const size_t row = 4 + (size_t)t.nm;
         std::vector<double> ord((t.nq + 2) * row, 0.0);
         std::vector<int32_t> sgn(t.nq + 8, 0);
+        auto tame = [](double x) { return x == 0.0 || (fabs(x) >= 1e-20 && fabs(x) <= 16.0); };
+        ctx->tameOrdinates = true;
         for (int q = 0; q < t.nq; ++q) {
+            if (!(tame(t.xi[q]) && tame(t.eta[q]) && tame(t.mu[q]) && tame(t.w[q])))
+                ctx->tameOrdinates = false;
             const double dir[3] = {t.xi[q], t.eta[q], t.mu[q]};
             double *r = ord.data() + q * row;
             for (int a = 0; a < 3; ++a) {
@@ -687,7 +691,7 @@ int c3d_flux_kinetic(c3d_ctx ctx, int nx, int ny, int nz, const double *alpha, d
         return C3D_ERR_HIP;
     hipStream_t s = (hipStream_t)stream;
     double *A = (double *)ctx->ansatz.p;
-    hipError_t e = launch_ansatz(ctx, nx, ny, nz, alpha, A, isPn, s);
+    hipError_t e = launch_ansatz(ctx, nx, ny, nz, alpha, A, isPn, dx, dy, dz, s);
     if (e == hipSuccess)
         e = launch_stencil(ctx, nx, ny, nz, A, flux, nullptr, nullptr, nullptr, 0.0, dx, dy, dz,
                            theta, 0, 0, s);
@@ -760,12 +764,12 @@ int c3d_update(c3d_ctx ctx, int nx, int ny, int nz, double *u, double *alpha,
             e = launch_closure_fp64(ctx, (int64_t)ng, u, alpha, oc,
                                     stats ? stats + st * ng : nullptr, s);
             if (e == hipSuccess)
-                e = launch_ansatz(ctx, nx, ny, nz, alpha, A, 0, s);
+                e = launch_ansatz(ctx, nx, ny, nz, alpha, A, 0, dx, dy, dz, s);
             if (e == hipSuccess)
                 e = launch_stencil(ctx, nx, ny, nz, A, nullptr, u, sigmaT, sigmaS, dt, dx, dy, dz,
                                    theta, 1, 0, s);
         } else {
-            e = launch_ansatz(ctx, nx, ny, nz, u, A, 1, s);
+            e = launch_ansatz(ctx, nx, ny, nz, u, A, 1, dx, dy, dz, s);
             if (e == hipSuccess)
                 e = launch_stencil(ctx, nx, ny, nz, A, nullptr, u, sigmaT, sigmaS, dt, dx, dy, dz,
                                    theta, 1, 0, s);
@@ -974,7 +978,8 @@ void solveFluxKinetic_hip(int nx, int ny, int nz, int nm, int nq, double dx, dou
         e = grow(g_f_ctx->ansatz, ng * nq * sizeof(double));
         double *A = (double *)g_f_ctx->ansatz.p;
         if (e == hipSuccess)
-            e = launch_ansatz(g_f_ctx, ix, iy, iz, (const double *)g_f_alpha.p, A, isPn, nullptr);
+            e = launch_ansatz(g_f_ctx, ix, iy, iz, (const double *)g_f_alpha.p, A, isPn, dx, dy, dz,
+                              nullptr);
         // theta = 2, as src/cuda/cuda_flux_kinetic.cu:82 hard-codes it
         if (e == hipSuccess)
             e = launch_stencil(g_f_ctx, ix, iy, iz, A, (double *)g_f_flux.p, nullptr, nullptr,

@@ -155,13 +155,14 @@ __device__ __forceinline__ void use_s(const double (&x)[N])
 // unit (the argument without FMA contraction, then exp) and the store of A.  M's rows are
 // uniform and come as scalar operands, half a row ahead; from LDS they took longer than the
 // vector work at M_4.  Small grids share out the ordinates over the blocks.
-// *wild is set where a value is not a number or exceeds kTame (see k_stencil).
+// *wild is set where a value is not a number, exceeds kTame, or is not zero but below tiny (see
+// k_stencil).
 constexpr double kTame = 1e290;
 template <int NM>
 __global__ __launch_bounds__(kTB) void k_ansatz(int64_t ng, int nq, int nqPer,
                                                  const double *__restrict__ ord,
                                                  const double *__restrict__ alpha, double *A,
-                                                 int isPn, int *wild)
+                                                 int isPn, double tiny, int *wild)
 {
     constexpr int HA = (NM + 1) / 2, HB = NM - HA;
     const int64_t cell = (int64_t)blockIdx.x * kTB + threadIdx.x;
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(kTB) void k_ansatz(int64_t ng, int nq, int nqPer,
         for (int m = 0; m < HB; ++m)
             kin += a[HA + m] * mB[m];
         const double v = isPn == 1 ? kin : (isPn == 2 ? det_exp(kin) : exp(kin));
-        bad |= !(fabs(v) <= kTame);
+        bad |= !(fabs(v) <= kTame) || (fabs(v) < tiny && v != 0.0);
         if (have)
             *At = v;
         At += ng;
@@ -261,6 +262,12 @@ bool exact_reciprocal(double d)
     int e = 0;
     return d > 0.0 && std::isfinite(d) && std::frexp(d, &e) == 0.5 && e > -1021 && e < 1022;
 }
+bool exact_reciprocals(double dx, double dy, double dz)
+{
+    return exact_reciprocal(dx) && exact_reciprocal(dy) && exact_reciprocal(dz);
+}
+// the least magnitude of the ansatz that k_stencil's fast path takes
+constexpr double kTinyDiv = 1e-200, kTinyP2 = 1e-270;
 
 typedef const __attribute__((address_space(1))) double GlobalDouble;
 typedef const __attribute__((address_space(1))) char GlobalByte;
@@ -317,9 +324,16 @@ __device__ __forceinline__ double div_by(double x, double d, double r)
 //     grids that leave the chip mostly idle;
 //   - the ordinate table as scalar operands, issued a stage ahead;
 //   - the tiling above, for the L2.
-// All of it gives the general path's bits as long as the ansatz is at most kTame, spacings and
-// theta are within reason and (Markstein) no axis's flux is below 1e-290; a NaN or a larger
-// value anywhere (*wild, from k_ansatz) sends the whole call down the general path.
+// All of it gives the general path's bits as long as the ansatz is zero or within [tiny, kTame]
+// and spacings, theta and the ordinates are within reason (launch_stencil): a value outside of
+// that, or a NaN, anywhere (*wild, from k_ansatz) sends the whole call down the general path.
+//
+// Why tiny: every difference of ansatz values is a multiple of e = ulp(tiny), and a limited
+// slope one of e / 2 (theta = 1) or of 2^-53 |theta| e, so that an axis's flux is zero or at
+// least a quarter of that times |direction| and weight.  With |theta| >= 1e-15 and directions
+// and weights >= 1e-20, tiny = 1e-200 leaves it above 1e-290, where div_by's residual is exact;
+// without a division (P2), 1e-270 keeps the slopes' factors of two exact.
+//
 // Measured, ansatz and stencil together, against a kernel with 13 loads, the nested limiter and
 // divisions: M_3 Q = 12 61x45x77 theta = 2: 945 -> 760 us; 96x128x128: 5.80 -> 4.60 ms; 16x12x20:
 // 535 -> 220 us; M_2 20^3 step, flux share: 220 -> 80 us.  The vector unit is busy 56% of the
@@ -891,8 +905,9 @@ hipError_t launch_ghost_fill(int nx, int ny, int nz, int nm, double *u, hipStrea
 }
 
 hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *alpha, double *A,
-                         int isPn, hipStream_t s)
+                         int isPn, double dx, double dy, double dz, hipStream_t s)
 {
+    const double tiny = exact_reciprocals(dx, dy, dz) ? kTinyP2 : kTinyDiv;
     // kind: 1 linear (P_N), 2 deterministic exp (reference-order mode), 0 device exp
     if (!isPn && ctx->precision == C3D_PREC_FP64_REFORDER)
         isPn = 2;
@@ -907,7 +922,7 @@ hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *a
     hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, ctx->d_wild);
 #define C3D_ANSATZ(NMV)                                                                        \
     hipLaunchKernelGGL(k_ansatz<NMV>, grid, dim3(kTB), 0, s, ng, nq, nqPer, ctx->d_ord, \
-                       alpha, A, isPn, ctx->d_wild)
+                       alpha, A, isPn, tiny, ctx->d_wild)
     switch (ctx->t.nm) {
     case 4: C3D_ANSATZ(4); break;
     case 9: C3D_ANSATZ(9); break;
@@ -928,9 +943,9 @@ hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *
     StencilArgs S{make_grid(nx, ny, nz), ctx->t.nq, dx, dy, dz, theta, dt, fuseEuler,
                   1.0 / dx, 1.0 / dy, 1.0 / dz, 0};
     // a plane's offsets are 32 bits of bytes on the fast path
-    S.general = !(tame(dx) && tame(dy) && tame(dz) && fabs(theta) < 1e15 &&
-                  (int64_t)S.G.NY * S.G.NZ < (1 << 29));
-    const bool p2 = exact_reciprocal(dx) && exact_reciprocal(dy) && exact_reciprocal(dz);
+    S.general = !(tame(dx) && tame(dy) && tame(dz) && (theta == 0.0 || tame(theta)) &&
+                  ctx->tameOrdinates && (int64_t)S.G.NY * S.G.NZ < (1 << 29));
+    const bool p2 = exact_reciprocals(dx, dy, dz);
     const bool th1 = theta == 1.0;
     dim3 grid(tile_blocks(S.G));
     // four ordinates in flight where there is at most a wave per SIMD
@@ -978,7 +993,7 @@ hipError_t launch_moment_stage(c3d_ctx_s *ctx, int nx, int ny, int nz, const dou
                                double dx, double dy, double dz, hipStream_t s)
 {
     Grid G = make_grid(nx, ny, nz);
-    const bool p2 = exact_reciprocal(dx) && exact_reciprocal(dy) && exact_reciprocal(dz);
+    const bool p2 = exact_reciprocals(dx, dy, dz);
     dim3 grid(tile_blocks(G));
 #define C3D_MOMENT(NMV)                                                                        \
     if (p2)                                                                                    \
