@@ -24,59 +24,12 @@
 
 #include "c3d_detmath.h"
 #include "c3d_internal.h"
+#include "c3d_tile.h"
 
 #pragma clang fp contract(off)
 
 namespace c3d {
 namespace {
-
-constexpr int kTB = 256;
-
-struct Grid {
-    int nx, ny, nz;
-    int NX, NY, NZ;  // with ghosts
-    __host__ __device__ size_t idx(int i, int j, int k) const
-    {
-        return (size_t)k + (size_t)NZ * ((size_t)j + (size_t)NY * (size_t)i);
-    }
-};
-
-Grid make_grid(int nx, int ny, int nz) { return Grid{nx, ny, nz, nx + 4, ny + 4, nz + 4}; }
-
-// ---------------------------------------------------------------- tiling of the interior
-// The stencil kernels give a block kTB consecutive cells of one x-plane's flattened (y, z)
-// interior, and order the blocks so that what one XCD has in flight is compact: block b goes
-// to XCD b % 8, so XCD x takes the x-th eighth of an order that walks strips of kStrip such
-// chunks along x.  A strip's planes are then fetched into that XCD's L2 once and reused by
-// the four planes after them; dealing consecutive chunks over the XCDs instead makes every
-// L2 fetch its own copy of the y and x neighbours.
-constexpr int kXcd = 8;
-constexpr int kStrip = 16;
-__host__ __device__ __forceinline__ int64_t plane_chunks(const Grid &G)
-{
-    return ((int64_t)G.ny * G.nz + kTB - 1) / kTB;
-}
-unsigned tile_blocks(const Grid &G)
-{
-    return (unsigned)((plane_chunks(G) * G.nx + kXcd - 1) / kXcd * kXcd);
-}
-struct Tile {
-    int i;      // x index of the block's plane, ghosts counted
-    int64_t p;  // first cell of the flattened interior plane
-};
-__device__ __forceinline__ bool tile_of(const Grid &G, Tile &t)
-{
-    const int64_t nP = plane_chunks(G), total = nP * G.nx;
-    const int64_t b = (int64_t)(blockIdx.x % kXcd) * (gridDim.x / kXcd) + blockIdx.x / kXcd;
-    if (b >= total)
-        return false;
-    const int64_t strip = b / (kStrip * (int64_t)G.nx);
-    const int64_t rem = b - strip * kStrip * G.nx;
-    const int64_t width = nP - strip * kStrip < kStrip ? nP - strip * kStrip : kStrip;
-    t.i = 2 + (int)(rem / width);
-    t.p = (strip * kStrip + rem % width) * kTB;
-    return true;
-}
 
 // ---------------------------------------------------------------- ghost fill
 // u2, if not null, receives the same ghosts
@@ -349,23 +302,25 @@ __global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__
     constexpr int OR = ord_row(NM);
     const Grid &G = S.G;
     Tile T;
-    if (!tile_of(G, T))
+    if (!tile_of(G, blockIdx.x, gridDim.x, blockDim.x, T))
         return;
-    const int64_t np = (int64_t)G.ny * G.nz;
-    const int64_t p = T.p + threadIdx.x;
-    const bool have = p < np;
-    // lanes past the plane's end work on its last cell and write nothing
-    const int64_t pc = have ? p : np - 1;
-    const int j = 2 + (int)(pc / G.nz), k = 2 + (int)(pc % G.nz);
+    // lanes past the run's end work on its last cell and write nothing; waves past it leave
+    const TileCell tc = tile_cell(G, T, threadIdx.x);
+    const bool have = tc.have;
+    if (__ballot(have) == 0)
+        return;
     const size_t ng = (size_t)G.NX * G.NY * G.NZ;
-    const size_t c = G.idx(T.i, j, k);
+    const size_t c = G.idx(T.i + tc.di, tc.j, tc.k);
     const ptrdiff_t sx = (ptrdiff_t)G.NY * G.NZ, sy = G.NZ;
     double fl[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m)
         fl[m] = 0.0;
     if (!S.general && *wild == 0) {
-        const unsigned inPlane = 8u * ((unsigned)j * (unsigned)G.NZ + (unsigned)k);
+        // bytes from the first cell's plane
+        const unsigned inPlane =
+            8u * (((unsigned)tc.di * (unsigned)G.NY + (unsigned)tc.j) * (unsigned)G.NZ +
+                  (unsigned)tc.k);
         const double *plane = A + (size_t)T.i * sx;
         // the values of the ordinate at plane b whose direction signs are sg (bits x, y, z; set:
         // positive)
@@ -548,6 +503,12 @@ struct OpRun {
     op8 lo, hi;
 };
 
+template <int NM, int KIND>
+constexpr int moment_lds()
+{
+    return kWave * ((NM | 1) + (KIND == kMomFlux ? 0 : 2));
+}
+
 // One thread per interior cell.  Bound by the vector unit (six NM x NM products without FMA
 // contraction) and, close behind, by HBM.  A lane that reads its own cell's moments touches a
 // cache line of its own per load (36 lines a load at nm = 9, which bound the kernel), so each
@@ -571,19 +532,19 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(NM <= 9 ? 3
                                                        const double *__restrict__ sigS)
 {
     constexpr int NMS = NM | 1;  // odd row stride: no bank conflicts reading a row per lane
-    __shared__ double sB[kTB / kWave][kWave * NMS];
-    __shared__ double sD[kTB / kWave][KIND == kMomFlux ? 1 : 2 * kWave];
+    extern __shared__ double sMem[];  // moment_lds<NM, KIND>() doubles a wave
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    double *const buf = sB[wv];
+    double *const buf = sMem + wv * moment_lds<NM, KIND>();
+    double *const sD = buf + kWave * NMS;  // the Euler factors
     Tile T;
-    if (!tile_of(G, T))
+    if (!tile_of(G, blockIdx.x, gridDim.x, blockDim.x, T))
         return;
-    // lanes past the plane's end work on its last cell and write nothing
-    const int64_t np = (int64_t)G.ny * G.nz;
-    const int64_t p = T.p + threadIdx.x;
-    const bool have = p < np;
-    const int64_t pc = have ? p : np - 1;
-    const size_t c = G.idx(T.i, 2 + (int)(pc / G.nz), 2 + (int)(pc % G.nz));
+    // lanes past the run's end work on its last cell and write nothing; waves past it leave
+    const TileCell tc = tile_cell(G, T, threadIdx.x);
+    const bool have = tc.have;
+    if (__ballot(have) == 0)
+        return;
+    const size_t c = G.idx(T.i + tc.di, tc.j, tc.k);
     const size_t c0 = (size_t)uniform_i64((long long)c);
     // element lane + 64 k of the wave's run: its place in memory, in bytes from the first cell's
     // moments (64 interior cells lie within a few rows or, where the rows are short, planes)
@@ -702,8 +663,8 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(NM <= 9 ? 3
     wave_lds_sync();
     if constexpr (KIND != kMomFlux) {  // the Euler factors of the lane's cell, update.cpp:28-35
         const double st = sigT[c], ss = sigS[c];
-        sD[wv][2 * lane] = 1.0 + dt * ss - dt * st;
-        sD[wv][2 * lane + 1] = 1.0 - dt * st;
+        sD[2 * lane] = 1.0 + dt * ss - dt * st;
+        sD[2 * lane + 1] = 1.0 - dt * st;
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m)
@@ -717,7 +678,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(NM <= 9 ? 3
         const int e = lane + kWave * k, l = e / NM;
         double v = buf[place(k)];
         if constexpr (KIND != kMomFlux)
-            v = el(run(0), rel[k]) * sD[wv][2 * l + (e - l * NM ? 1 : 0)] - dt * v;
+            v = el(run(0), rel[k]) * sD[2 * l + (e - l * NM ? 1 : 0)] - dt * v;
         if constexpr (KIND == kMomStage2)
             v = 0.5 * (v + el(at, rel[k]));
         if (e < nHave)
@@ -942,21 +903,22 @@ hipError_t launch_stencil(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *
     auto tame = [](double x) { return fabs(x) > 1e-15 && fabs(x) < 1e15; };
     StencilArgs S{make_grid(nx, ny, nz), ctx->t.nq, dx, dy, dz, theta, dt, fuseEuler,
                   1.0 / dx, 1.0 / dy, 1.0 / dz, 0};
-    // a plane's offsets are 32 bits of bytes on the fast path
+    // a block's offsets within its planes are 32 bits of bytes on the fast path
     S.general = !(tame(dx) && tame(dy) && tame(dz) && (theta == 0.0 || tame(theta)) &&
                   ctx->tameOrdinates && (int64_t)S.G.NY * S.G.NZ < (1 << 29));
     const bool p2 = exact_reciprocals(dx, dy, dz);
     const bool th1 = theta == 1.0;
-    dim3 grid(tile_blocks(S.G));
+    const int tb = tile_threads(S.G, ctx->numCU);
+    dim3 grid(tile_blocks(S.G, tb));
     // four ordinates in flight where there is at most a wave per SIMD
-    const bool deep = grid.x <= (unsigned)ctx->numCU;
+    const bool deep = tb < kTB;
     if (zeroGhosts && !fuseEuler) {
         const int64_t ng = (int64_t)S.G.NX * S.G.NY * S.G.NZ;
         hipLaunchKernelGGL(k_zero_ghost_flux, dim3(blocks_for(ng * ctx->t.nm, 256, 65536)),
                            dim3(256), 0, s, S.G, ctx->t.nm, flux);
     }
 #define C3D_STENCIL_V(NMV, P, T, D)                                                           \
-    hipLaunchKernelGGL((k_stencil<NMV, P, T, D>), grid, dim3(kTB), 0, s, S, A, ctx->d_ord,     \
+    hipLaunchKernelGGL((k_stencil<NMV, P, T, D>), grid, dim3(tb), 0, s, S, A, ctx->d_ord,     \
                        ctx->d_sgn, ctx->d_wild, flux, u, sigmaT, sigmaS)
 #define C3D_STENCIL_D(NMV, D)                                                                 \
     if (p2 && th1)                                                                             \
@@ -994,14 +956,17 @@ hipError_t launch_moment_stage(c3d_ctx_s *ctx, int nx, int ny, int nz, const dou
 {
     Grid G = make_grid(nx, ny, nz);
     const bool p2 = exact_reciprocals(dx, dy, dz);
-    dim3 grid(tile_blocks(G));
+    const int tb = tile_threads(G, ctx->numCU);
+    dim3 grid(tile_blocks(G, tb));
+#define C3D_MOMENT_V(NMV, P)                                                                   \
+    hipLaunchKernelGGL((k_moment_stage<NMV, KIND, P>), grid, dim3(tb),                         \
+                       (tb / kWave * moment_lds<NMV, KIND>() * sizeof(double)), s, G, src, dst,\
+                       ctx->d_pnOps, dx, dy, dz, dt, sigmaT, sigmaS)
 #define C3D_MOMENT(NMV)                                                                        \
     if (p2)                                                                                    \
-        hipLaunchKernelGGL((k_moment_stage<NMV, KIND, true>), grid, dim3(kTB), 0, s, G, src,   \
-                           dst, ctx->d_pnOps, dx, dy, dz, dt, sigmaT, sigmaS);                 \
+        C3D_MOMENT_V(NMV, true);                                                               \
     else                                                                                       \
-        hipLaunchKernelGGL((k_moment_stage<NMV, KIND, false>), grid, dim3(kTB), 0, s, G, src,  \
-                           dst, ctx->d_pnOps, dx, dy, dz, dt, sigmaT, sigmaS)
+        C3D_MOMENT_V(NMV, false)
     switch (ctx->t.nm) {
     case 4: C3D_MOMENT(4); break;
     case 9: C3D_MOMENT(9); break;
@@ -1010,6 +975,7 @@ hipError_t launch_moment_stage(c3d_ctx_s *ctx, int nx, int ny, int nz, const dou
     default: return hipErrorInvalidValue;
     }
 #undef C3D_MOMENT
+#undef C3D_MOMENT_V
     return hipGetLastError();
 }
 }  // namespace
