@@ -22,7 +22,7 @@ inline Grid make_grid(int nx, int ny, int nz)
     return Grid{nx, ny, nz, nx + 4, ny + 4, nz + 4};
 }
 
-// A block of tb threads works on tb consecutive cells of a run of flattened interior cells (z
+// A block of tb threads (a power of two) works on tb consecutive cells of a run of flattened interior cells (z
 // fastest).  Block b goes to XCD b % kXcd, and XCD x takes the x-th eighth of an order of the
 // blocks that keeps compact what it has in flight, so that a plane is fetched into that XCD's L2
 // once and reused by the four planes after it; dealing consecutive blocks over the XCDs instead
@@ -44,7 +44,7 @@ __host__ __device__ inline bool flat_tiles(const Grid &G) { return plane_cells(G
 __host__ __device__ inline int64_t tile_count(const Grid &G, int tb)
 {
     const int64_t run = flat_tiles(G) ? plane_cells(G) * G.nx : plane_cells(G);
-    const int64_t n = (run + tb - 1) / tb;
+    const int64_t n = (run + tb - 1) >> __builtin_ctz(tb);
     return flat_tiles(G) ? n : n * G.nx;
 }
 inline unsigned tile_blocks(const Grid &G, int tb)
@@ -63,22 +63,22 @@ struct Tile {
 __host__ __device__ inline bool tile_of(const Grid &G, unsigned block, unsigned blocks, int tb,
                                         Tile &t)
 {
-    const int64_t b = (int64_t)(block % kXcd) * (blocks / kXcd) + block / kXcd;
+    // a launch has fewer than 2^32 threads, so that blocks and cells are counted in 32 bits
+    const unsigned b = block % kXcd * (blocks / kXcd) + block / kXcd;
     if (b >= tile_count(G, tb))
         return false;
-    const int64_t P = plane_cells(G);
+    const unsigned P = (unsigned)plane_cells(G), sh = __builtin_ctz(tb);
     if (flat_tiles(G)) {
-        const int64_t c = b * tb, i = c / P;
+        const unsigned c = b << sh, i = c / P;
         t.i = 2 + (int)i;
         t.p = c - i * P;
         return true;
     }
-    const int64_t nP = (P + tb - 1) / tb, nS = kStripCells / tb;
-    const int64_t strip = b / (nS * G.nx);
-    const int64_t rem = b - strip * nS * G.nx;
-    const int64_t width = nP - strip * nS < nS ? nP - strip * nS : nS;
+    const unsigned nP = (P + tb - 1) >> sh, nS = kStripCells >> sh;
+    const unsigned strip = b / (nS * G.nx), rem = b - strip * nS * G.nx;
+    const unsigned width = nP - strip * nS < nS ? nP - strip * nS : nS;
     t.i = 2 + (int)(rem / width);
-    t.p = (strip * nS + rem % width) * tb;
+    t.p = (int64_t)(strip * nS + rem % width) << sh;
     return true;
 }
 
@@ -91,7 +91,6 @@ struct TileCell {
 };
 __host__ __device__ inline TileCell tile_cell(const Grid &G, const Tile &T, int lane)
 {
-    // a grid whose plane has 2^32 cells does not fit the card
     const unsigned P = (unsigned)plane_cells(G);
     unsigned r = (unsigned)T.p + (unsigned)lane, di = 0;
     bool have = r < P;
