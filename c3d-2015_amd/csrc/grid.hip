@@ -6,8 +6,10 @@
 //   k_stencil      limited upwind differences, sum_q m_q (Fx/dx+Fy/dy+Fz/dz), optionally
 //                  fused with the Euler stage             flux_kinetic.cpp:45-60, 126-196,
 //                                                        update.cpp:21-37
-//   k_moment_stage P_N Fromm flux with half-range operators, alone or with the Euler stage
-//                  and the RK2 average                    flux_moment.cpp:30-104,
+//   k_flux_moment  P_N Fromm flux with half-range operators (nm <= 9)
+//                                                        flux_moment.cpp:30-104
+//   k_moment_stage the same flux, alone (nm > 9) or with the Euler stage and the RK2 average
+//                                                        flux_moment.cpp:30-104,
 //                                                        update.cpp:21-37, 268-274
 //   k_euler        Euler stage with isotropic scattering update.cpp:21-37
 //   k_rk2          uOld <- u / u <- (u + uOld)/2          update.cpp:206-212, 268-274
@@ -503,6 +505,67 @@ struct OpRun {
     op8 lo, hi;
 };
 
+// The flux alone up to nm = 9, one thread per interior cell on its own moments, the operators'
+// columns broadcast from LDS.  k_moment_stage's runs, LDS turns and scalar operands are a longer
+// chain of waits, which pays where they save the passes of a whole step and from nm = 16 on, but
+// not here.  Measured, k_moment_stage -> this: P_1 64^3 12.4 -> 10.7 us, 128^3 65 -> 51; P_2 20^3
+// 15.8 -> 11.2, 64^3 34 -> 31, 80^3 65 -> 51, 128^3 271 -> 211.
+template <int NM>
+__global__ __launch_bounds__(kTB) void k_flux_moment(Grid G, const double *__restrict__ u,
+                                                      double *flux,
+                                                      const double *__restrict__ opsT, double dx,
+                                                      double dy, double dz)
+{
+    __shared__ double sO[6 * NM * NM];
+    for (int e = threadIdx.x; e < 6 * NM * NM; e += blockDim.x)
+        sO[e] = opsT[e];
+    __syncthreads();
+    Tile T;
+    if (!tile_of(G, blockIdx.x, gridDim.x, blockDim.x, T))
+        return;
+    const TileCell tc = tile_cell(G, T, threadIdx.x);
+    if (!tc.have)
+        return;
+    const size_t c = G.idx(T.i + tc.di, tc.j, tc.k);
+    const size_t strides[3] = {(size_t)G.NY * G.NZ, (size_t)G.NZ, 1};
+    const double hs[3] = {dx, dy, dz};
+    double out[NM];
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        const size_t s = strides[ax];
+        const double *um2 = u + (c - 2 * s) * NM, *um1 = u + (c - s) * NM, *u0 = u + c * NM,
+                     *up1 = u + (c + s) * NM, *up2 = u + (c + 2 * s) * NM;
+        const double *Op = sO + (2 * ax) * NM * NM, *Om = Op + NM * NM;
+        double temp[NM], F[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+            temp[m] = 0.25 * up1[m] + 0.75 * u0[m] - 1.25 * um1[m] + 0.25 * um2[m];
+#pragma unroll
+        for (int r = 0; r < NM; ++r)
+            F[r] = 0.0;
+#pragma unroll
+        for (int q = 0; q < NM; ++q)
+#pragma unroll
+            for (int r = 0; r < NM; ++r)
+                F[r] += Op[q * NM + r] * temp[q];
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+            temp[m] = -0.25 * up2[m] + 1.25 * up1[m] - 0.75 * u0[m] - 0.25 * um1[m];
+#pragma unroll
+        for (int q = 0; q < NM; ++q)
+#pragma unroll
+            for (int r = 0; r < NM; ++r)
+                F[r] += Om[q * NM + r] * temp[q];
+        // flux = xF/dx + yF/dy + zF/dz, accumulated left to right
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+            out[m] = ax == 0 ? F[m] / hs[0] : out[m] + F[m] / hs[ax];
+    }
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+        flux[c * NM + m] = out[m];
+}
+
 template <int NM, int KIND>
 constexpr int moment_lds()
 {
@@ -967,9 +1030,13 @@ hipError_t launch_moment_stage(c3d_ctx_s *ctx, int nx, int ny, int nz, const dou
         C3D_MOMENT_V(NMV, true);                                                               \
     else                                                                                       \
         C3D_MOMENT_V(NMV, false)
+    if constexpr (KIND != kMomFlux) {  // k_flux_moment's
+        switch (ctx->t.nm) {
+        case 4: C3D_MOMENT(4); return hipGetLastError();
+        case 9: C3D_MOMENT(9); return hipGetLastError();
+        }
+    }
     switch (ctx->t.nm) {
-    case 4: C3D_MOMENT(4); break;
-    case 9: C3D_MOMENT(9); break;
     case 16: C3D_MOMENT(16); break;
     case 25: C3D_MOMENT(25); break;
     default: return hipErrorInvalidValue;
@@ -983,8 +1050,18 @@ hipError_t launch_moment_stage(c3d_ctx_s *ctx, int nx, int ny, int nz, const dou
 hipError_t launch_flux_moment(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *u,
                               double *flux, double dx, double dy, double dz, hipStream_t s)
 {
-    return launch_moment_stage<kMomFlux>(ctx, nx, ny, nz, u, flux, nullptr, nullptr, 0.0, dx, dy,
-                                         dz, s);
+    if (ctx->t.nm > 9)
+        return launch_moment_stage<kMomFlux>(ctx, nx, ny, nz, u, flux, nullptr, nullptr, 0.0, dx,
+                                             dy, dz, s);
+    Grid G = make_grid(nx, ny, nz);
+    dim3 grid(tile_blocks(G, kTB));
+    if (ctx->t.nm == 4)
+        hipLaunchKernelGGL(k_flux_moment<4>, grid, dim3(kTB), 0, s, G, u, flux, ctx->d_pnOps, dx,
+                           dy, dz);
+    else
+        hipLaunchKernelGGL(k_flux_moment<9>, grid, dim3(kTB), 0, s, G, u, flux, ctx->d_pnOps, dx,
+                           dy, dz);
+    return hipGetLastError();
 }
 
 // one SSP-RK2 step of the P_N equations with the moment flux; b: a grid's worth of scratch
