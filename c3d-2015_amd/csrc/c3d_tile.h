@@ -106,4 +106,14 @@ __host__ __device__ inline TileCell tile_cell(const Grid &G, const Tile &T, int 
     return TileCell{(int)di, 2 + (int)j, 2 + (int)(r - j * (unsigned)G.nz), have};
 }
 
+// Whether a stencil (two cells each way along each axis, from an interior cell) reads the cell: not
+// if two or three of its coordinates are ghosts'.  Those cells are never filled.
+__host__ __device__ inline bool stencil_reads(const Grid &G, unsigned cell)
+{
+    const unsigned row = cell / (unsigned)G.NZ, plane = row / (unsigned)G.NY;
+    const int k = (int)(cell - row * (unsigned)G.NZ), j = (int)(row - plane * (unsigned)G.NY),
+              i = (int)plane;
+    return (i < 2 || i >= G.nx + 2) + (j < 2 || j >= G.ny + 2) + (k < 2 || k >= G.nz + 2) <= 1;
+}
+
 }  // namespace c3d

@@ -111,10 +111,10 @@ __device__ __forceinline__ void use_s(const double (&x)[N])
 // uniform and come as scalar operands, half a row ahead; from LDS they took longer than the
 // vector work at M_4.  Small grids share out the ordinates over the blocks.
 // *wild is set where a value is not a number, exceeds kTame, or is not zero but below tiny (see
-// k_stencil).
+// k_stencil), in a cell that some stencil reads.
 constexpr double kTame = 1e290;
 template <int NM>
-__global__ __launch_bounds__(kTB) void k_ansatz(int64_t ng, int nq, int nqPer,
+__global__ __launch_bounds__(kTB) void k_ansatz(Grid G, int64_t ng, int nq, int nqPer,
                                                  const double *__restrict__ ord,
                                                  const double *__restrict__ alpha, double *A,
                                                  int isPn, double tiny, int *wild)
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kTB) void k_ansatz(int64_t ng, int nq, int nqPer,
             *At = v;
         At += ng;
     }
-    if (have && bad)
+    if (have && bad && stencil_reads(G, (unsigned)cell))
         *wild = 1;
 }
 __global__ void k_clear_int(int *p) { *p = 0; }
@@ -293,8 +293,10 @@ __device__ __forceinline__ double div_by(double x, double d, double r)
 // divisions: M_3 Q = 12 61x45x77 theta = 2: 945 -> 760 us; 96x128x128: 5.80 -> 4.60 ms; 16x12x20:
 // 535 -> 220 us; M_2 20^3 step, flux share: 220 -> 80 us.  The vector unit is busy 56% of the
 // large grid's time (855 M instructions); the L1 serves 10 unaligned rows per cell and ordinate.
+// The fast path's registers set the waves of a SIMD (D = 2); the general path gets by with them.
+constexpr int stencil_waves(int nm, int d) { return d > 2 ? 1 : (nm == 4 ? 6 : (nm == 9 ? 5 : 4)); }
 template <int NM, bool P2, bool TH1, int D>
-__global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__restrict__ A,
+__global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(stencil_waves(NM, D)))) void k_stencil(StencilArgs S, const double *__restrict__ A,
                                                   const double *__restrict__ ord,
                                                   const int *__restrict__ sgn,
                                                   const int *__restrict__ wild, double *flux,
@@ -302,9 +304,10 @@ __global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__
                                                   const double *__restrict__ sigS)
 {
     constexpr int OR = ord_row(NM);
+    constexpr int TB = D > 2 ? kTBSmall : kTB;  // as launched
     const Grid &G = S.G;
     Tile T;
-    if (!tile_of(G, blockIdx.x, gridDim.x, blockDim.x, T))
+    if (!tile_of(G, blockIdx.x, gridDim.x, TB, T))
         return;
     // lanes past the run's end work on its last cell and write nothing; waves past it leave
     const TileCell tc = tile_cell(G, T, threadIdx.x);
@@ -312,22 +315,20 @@ __global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__
     if (__ballot(have) == 0)
         return;
     const size_t ng = (size_t)G.NX * G.NY * G.NZ;
-    const size_t c = G.idx(T.i + tc.di, tc.j, tc.k);
+    // cells from the start of the tile's first plane
+    const unsigned in =
+        ((unsigned)tc.di * (unsigned)G.NY + (unsigned)tc.j) * (unsigned)G.NZ + (unsigned)tc.k;
     const ptrdiff_t sx = (ptrdiff_t)G.NY * G.NZ, sy = G.NZ;
     double fl[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m)
         fl[m] = 0.0;
     if (!S.general && *wild == 0) {
-        // bytes from the first cell's plane
-        const unsigned inPlane =
-            8u * (((unsigned)tc.di * (unsigned)G.NY + (unsigned)tc.j) * (unsigned)G.NZ +
-                  (unsigned)tc.k);
         const double *plane = A + (size_t)T.i * sx;
         // the values of the ordinate at plane b whose direction signs are sg (bits x, y, z; set:
         // positive)
         auto load = [&](double(&v)[10], const double *b, int sg) {
-            unsigned off = inPlane;
+            unsigned off = 8u * in;
             asm("" : "+v"(off));  // widened here, next to the loads
             auto at = [&](ptrdiff_t o) {
                 // the base stays scalar: one register offset serves every load
@@ -433,14 +434,29 @@ __global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__
             }
         }
     } else {
+        // the 13 values of the cell's stencil: the centre, then -2, -1, +1, +2 along x, y and z;
+        // up to nm = 16 the next ordinate's are in flight while this one's are used (at nm = 25
+        // there are no registers for them beside the fast path's waves)
+        constexpr bool kAhead = NM <= 16;
+        const ptrdiff_t off[13] = {0,       -2 * sx, -sx, sx, 2 * sx, -2 * sy, -sy,
+                                   sy,      2 * sy,  -2,  -1, 1,      2};
+        const double *a = A + (size_t)T.i * sx + in, *row = ord;
+        double v[13], nv[13];
+#pragma unroll
+        for (int e = 0; e < 13; ++e)
+            v[e] = a[off[e]];
         for (int q = 0; q < S.nq; ++q) {
-            const double *a = A + (size_t)q * ng + c, *row = ord + (size_t)q * OR;
-            const double a0 = a[0], wq = row[3];
-            const double fX = axis_flux<TH1>(a[-2 * sx], a[-sx], a0, a[sx], a[2 * sx], row[0],
-                                             wq, S.theta);
-            const double fY = axis_flux<TH1>(a[-2 * sy], a[-sy], a0, a[sy], a[2 * sy], row[1],
-                                             wq, S.theta);
-            const double fZ = axis_flux<TH1>(a[-2], a[-1], a0, a[1], a[2], row[2], wq, S.theta);
+            a += q + 1 < S.nq ? ng : 0;
+            if constexpr (kAhead) {
+#pragma unroll
+                for (int e = 0; e < 13; ++e)
+                    nv[e] = a[off[e]];
+            }
+            const double wq = row[3];
+            const double fX = axis_flux<TH1>(v[1], v[2], v[0], v[3], v[4], row[0], wq, S.theta);
+            const double fY = axis_flux<TH1>(v[5], v[6], v[0], v[7], v[8], row[1], wq, S.theta);
+            const double fZ =
+                axis_flux<TH1>(v[9], v[10], v[0], v[11], v[12], row[2], wq, S.theta);
             double s;
             if constexpr (P2)
                 s = fX * S.rdx + fY * S.rdy + fZ * S.rdz;
@@ -449,18 +465,26 @@ __global__ __launch_bounds__(kTB) void k_stencil(StencilArgs S, const double *__
 #pragma unroll
             for (int m = 0; m < NM; ++m)
                 fl[m] += row[4 + m] * s;
+#pragma unroll
+            for (int e = 0; e < 13; ++e)
+                v[e] = kAhead ? nv[e] : a[off[e]];
+            row += OR;
         }
     }
     if (!have)
         return;
+    const size_t c = (size_t)T.i * sx + in;
     if (S.fuseEuler) {
         // update.cpp:28-35
         const double dt = S.dt, st = sigT[c], ss = sigS[c];
         double *uc = u + c * NM;
         uc[0] = uc[0] * (1.0 + dt * ss - dt * st) - dt * fl[0];
 #pragma unroll
-        for (int m = 1; m < NM; ++m)
+        for (int m = 1; m < NM; ++m) {
             uc[m] = uc[m] * (1.0 - dt * st) - dt * fl[m];
+            if (m % 12 == 0)  // not all of u in registers beside the flux
+                __builtin_amdgcn_sched_barrier(0);
+        }
     } else {
 #pragma unroll
         for (int m = 0; m < NM; ++m)
@@ -935,7 +959,8 @@ hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *a
     // kind: 1 linear (P_N), 2 deterministic exp (reference-order mode), 0 device exp
     if (!isPn && ctx->precision == C3D_PREC_FP64_REFORDER)
         isPn = 2;
-    const int64_t ng = (int64_t)(nx + 4) * (ny + 4) * (nz + 4);
+    const Grid G = make_grid(nx, ny, nz);
+    const int64_t ng = (int64_t)G.NX * G.NY * G.NZ;
     const int nq = ctx->t.nq;
     // small grids share out the ordinates too: 8 blocks a CU, at least 16 ordinates each
     const int64_t bx = blocks_for(ng, kTB, INT32_MAX);
@@ -945,7 +970,7 @@ hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *a
     dim3 grid((unsigned)bx, (unsigned)split);
     hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, ctx->d_wild);
 #define C3D_ANSATZ(NMV)                                                                        \
-    hipLaunchKernelGGL(k_ansatz<NMV>, grid, dim3(kTB), 0, s, ng, nq, nqPer, ctx->d_ord, \
+    hipLaunchKernelGGL(k_ansatz<NMV>, grid, dim3(kTB), 0, s, G, ng, nq, nqPer, ctx->d_ord, \
                        alpha, A, isPn, tiny, ctx->d_wild)
     switch (ctx->t.nm) {
     case 4: C3D_ANSATZ(4); break;

@@ -1,5 +1,6 @@
 // The stencil kernels' tiling (csrc/c3d_tile.h) on the host: nx ny nz threads -> blocks launched, or a
-// complaint if a cell is missed or taken twice, or a thread without one is given no valid cell.
+// complaint if a cell is missed or taken twice, or a thread without one is given no valid cell, or the
+// cells that stencils read are not those that they are said to read.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -45,5 +46,16 @@ int main(int argc, char **argv)
             for (int k = 2; k < G.nz + 2; ++k)
                 if (!seen[G.idx(i, j, k)])
                     return std::puts("a cell is missed"), 1;
+    // the cells that some interior cell's stencil reads
+    std::vector<char> read(seen.size(), 0);
+    for (int i = 2; i < G.nx + 2; ++i)
+        for (int j = 2; j < G.ny + 2; ++j)
+            for (int k = 2; k < G.nz + 2; ++k)
+                for (int o = -2; o <= 2; ++o)
+                    read[G.idx(i + o, j, k)] = read[G.idx(i, j + o, k)] =
+                        read[G.idx(i, j, k + o)] = 1;
+    for (size_t c = 0; c < read.size(); ++c)
+        if (c3d::stencil_reads(G, (unsigned)c) != (read[c] != 0))
+            return std::puts("a cell's use"), 1;
     std::printf("%u\n", blocks);
 }
