@@ -3780,18 +3780,21 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                 }
                 __syncthreads();
                 // The search over the verdicts in order: at trial k it accepts, or halves the
-                // step (ls_reject) and gives up if that is too short.  Lane k looks at trial k.
+                // step (ls_reject) and gives up if that is too short.  The first trial is accepted
+                // most often; beyond it lane k looks at trial k.
                 const int n = TW * kw;
                 static_assert(TW * KWA <= kWave, "a lane per trial");
-                const bool okK = lane < n && sOk[lane < n ? lane : 0];
-                const bool deadK =
-                    lane < n && !(ldexp(C.tls, -(lane + 1)) * C.maxF > DBL_EPSILON / 2);
-                const unsigned long long okM = __ballot(okK), deadM = __ballot(deadK);
-                const int kOk = okM ? __ffsll(okM) - 1 : n, kDead = deadM ? __ffsll(deadM) - 1 : n;
-                const bool accepted = kOk < n && kOk <= kDead;
-                if (accepted ? kOk > 0 : n > 0) {  // the last rejection, with its ls_next()
-                    const int last = accepted ? kOk : min(kDead + 1, n);
-                    C.tls = ldexp(C.tls, 1 - last);
+                bool accepted = sOk[0];
+                if (!accepted) {
+                    const bool okK = lane < n && sOk[lane < n ? lane : 0];
+                    const bool deadK =
+                        lane < n && !(ldexp(C.tls, -(lane + 1)) * C.maxF > DBL_EPSILON / 2);
+                    const unsigned long long okM = __ballot(okK), deadM = __ballot(deadK);
+                    const int kOk = okM ? __ffsll(okM) - 1 : n;
+                    const int kDead = deadM ? __ffsll(deadM) - 1 : n;
+                    accepted = kOk < n && kOk <= kDead;
+                    // the last rejection, with its ls_next()
+                    C.tls = ldexp(C.tls, 1 - (accepted ? kOk : min(kDead + 1, n)));
                     C.ls_reject(li);
                 }
                 __syncthreads();  // sOk and sA are rewritten by the next round
