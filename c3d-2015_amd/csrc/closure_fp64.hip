@@ -3454,11 +3454,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 // (one point).  (The mixed phase's points: f_trials_mixed.)  M is read from the transposed
 // table MT [NM][nqPad] (one coalesced load per component), each chunk's M shared by the points.
 // Bound by latency: the wave is alone on its SIMD, so all points' exponents and exps run side
-// by side, with few points those of two chunks (their terms are added in chunk order), and the
+// by side, with few points those of H = 2 chunks (their terms are added in chunk order), and the
 // next chunks are in flight meanwhile; the point count is a constant, since a test per point
 // would end each chain before the next starts.
 enum : int { kFp64 = 0, kFRef = 1 };
-template <int NM, int MODE, int KW>
+template <int NM, int MODE, int KW, int H = KW >= 4 ? 1 : 2>
 __device__ __forceinline__ void f_trials(const KParams &P, const double *__restrict__ MT,
                                          const double *__restrict__ wg, const double *sA,
                                          double *sW, double *sE, int lane, double (&out)[KW])
@@ -3489,8 +3489,7 @@ __device__ __forceinline__ void f_trials(const KParams &P, const double *__restr
     } else {
         // ordinate mfma_ordinate(lane) of each chunk, as chunk_mfma does; a chunk past the last
         // is the last one again, left out of the sum
-        constexpr int H = KW >= 4 ? 1 : 2;  // chunks side by side
-        constexpr int NB = KW >= 4 ? 2 : 1;  // and such groups in flight
+        constexpr int NB = H == 1 ? 2 : 1;  // groups of H chunks in flight
         struct Group {
             double m[H][NM], w[H];
         };
@@ -3665,6 +3664,9 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
     // points side by side: the mixed kernel at nm = 9 would spill with eight (M_2 closure of 3000
     // cells 2.87 -> 3.17 ms)
     constexpr int KB = MIXED && NM <= 9 ? 4 : KW;
+    // chunks side by side for a single point: two, but one in the FP64 kernel at nm = 16, whose
+    // chains are long enough (200 to 3000 M_3 cells 1% faster so, the other kernels slower)
+    constexpr int H1 = NM == 16 && !MIXED ? 1 : 2;
     // in the mixed phase the points are the rows of the exponent products: four per wave
     constexpr int KWM = 4;
     constexpr int KWA = MIXED && KWM > KW ? KWM : KW;
@@ -3748,7 +3750,8 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                         double fk[KW];
                         if (KW > 1 && kw == 1) {
                             double f1[1];
-                            f_trials<NM, MODE, 1>(P, MT, wg, sA[wv], sW[wv], sE[wv], lane, f1);
+                            f_trials<NM, MODE, 1, H1>(P, MT, wg, sA[wv], sW[wv], sE[wv], lane,
+                                                      f1);
 #pragma unroll
                             for (int j = 0; j < KW; ++j)
                                 fk[j] = j == 0 ? f1[0] : 0.0;
@@ -3780,11 +3783,12 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                 }
                 __syncthreads();
                 // The search over the verdicts in order: at trial k it accepts, or halves the
-                // step (ls_reject) and gives up if that is too short.  The first trial is accepted
-                // most often; beyond it lane k looks at trial k.
+                // step (ls_reject) and gives up if that is too short.  Lane k looks at trial k; up to
+                // nm = 16 only if the first one, accepted most often, is not (batches of 200 cells
+                // 1 to 2% faster so, the longer rounds of M_4 1% slower).
                 const int n = TW * kw;
                 static_assert(TW * KWA <= kWave, "a lane per trial");
-                bool accepted = sOk[0];
+                bool accepted = NM <= 16 && sOk[0];
                 if (!accepted) {
                     const bool okK = lane < n && sOk[lane < n ? lane : 0];
                     const bool deadK =
@@ -3793,9 +3797,10 @@ __global__ __launch_bounds__(TW * kWave) void k_tail(KParams P, const double *__
                     const int kOk = okM ? __ffsll(okM) - 1 : n;
                     const int kDead = deadM ? __ffsll(deadM) - 1 : n;
                     accepted = kOk < n && kOk <= kDead;
-                    // the last rejection, with its ls_next()
-                    C.tls = ldexp(C.tls, 1 - (accepted ? kOk : min(kDead + 1, n)));
-                    C.ls_reject(li);
+                    if (!accepted || kOk > 0) {  // the last rejection, with its ls_next()
+                        C.tls = ldexp(C.tls, 1 - (accepted ? kOk : min(kDead + 1, n)));
+                        C.ls_reject(li);
+                    }
                 }
                 __syncthreads();  // sOk and sA are rewritten by the next round
                 if (!accepted)
