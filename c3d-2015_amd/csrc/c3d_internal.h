@@ -94,7 +94,7 @@ struct c3d_ctx_s {
     c3d::ClosureConsts cc{};
     int nqPad = 0;  // nq rounded up to kChunk
     // device tables
-    double *d_w = nullptr, *d_xi = nullptr, *d_eta = nullptr, *d_mu = nullptr;
+    double *d_w = nullptr;
     double *d_ord = nullptr;   // [nq + 2][4 + nm], rows (xi, eta, mu, w, M's row); two zero rows
     int32_t *d_sgn = nullptr;  // [nq + 8], bits 0..2: xi, eta, mu > 0
     int *d_wild = nullptr;     // the ansatz holds a NaN, a huge or a tiny value (grid.hip)

@@ -84,9 +84,6 @@ int finish_ctx(c3d_ctx_s *ctx)
     if (e == hipSuccess)                                                                       \
     e = upload(&ctx->dst, vec.data(), vec.size())
     UP(d_w, t.w);
-    UP(d_xi, t.xi);
-    UP(d_eta, t.eta);
-    UP(d_mu, t.mu);
     UP(d_M, Mp);
     {
         std::vector<double> MTp((size_t)ctx->nqPad * t.nm, 0.0);
@@ -294,7 +291,7 @@ int c3d_destroy(c3d_ctx ctx)
 {
     if (!ctx)
         return C3D_OK;
-    void *ptrs[] = {ctx->d_w, ctx->d_xi, ctx->d_eta, ctx->d_mu, ctx->d_M, ctx->d_MT,
+    void *ptrs[] = {ctx->d_w, ctx->d_M, ctx->d_MT,
                     ctx->d_wpad, ctx->d_P16, ctx->d_R, ctx->d_M2, ctx->d_beta, ctx->d_betaVal, ctx->d_pnOps, ctx->d_betaColInd,
                     ctx->d_betaRowPtr, ctx->d_sweepCount, ctx->d_status, ctx->d_wild, ctx->d_ord, ctx->d_sgn, ctx->ansatz.p,
                     ctx->uOld.p, ctx->closureState.p};
