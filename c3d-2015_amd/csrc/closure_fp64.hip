@@ -12,14 +12,16 @@
 //            sum_q w_q e_q and H = M^T diag(w e) M.  A wavefront takes 4 cells; the block's
 //            16 cells share every M chunk staged in LDS, and the four cells' lower-triangle
 //            4x4 blocks of H accumulate on the matrix cores (V_MFMA_F64_4X4X4_4B_F64, one
-//            cell per block slot: Quad).  H is stored as its packed lower triangle.
+//            cell per block slot: Quad).  H is stored as those blocks (HBlock).
 //   k_step   advances each listed cell by exactly one step of its state machine with that
 //            sweep's result: either the Armijo test of a line-search trial, or one Newton
-//            iteration (Cholesky in dpotf2 order, the dlacn2/dtrsv condition estimate, the
-//            restart/ladder decisions, the solve of utils.cpp:71-86, dnrm2, modcfl, line-
-//            search setup).  Row i of H lives in lane i; every scalar is reduced in the
-//            CPU's sequential order without FMA contraction.  Unfinished cells append
-//            themselves to the next worklist.
+//            iteration (Cholesky, the dlacn2 condition estimate, the restart/ladder decisions,
+//            the solve of utils.cpp:71-86, dnrm2, modcfl, line-search setup).  A cell's rows are
+//            shared out over 4 lanes (16 at nm = 25), and reductions are trees (Rows).
+//            Unfinished cells append themselves to the next worklist.
+// The reference-order mode has k_sweep_ref and k_step_ref in their place: H row-major with both
+// triangles, row i in lane i, dpotf2's and dtrsv's order, and every scalar reduced in the CPU's
+// sequential order.  Multiply-adds are fused only where the code says so.
 // Every loop in both kernels is bounded by sizes fixed at launch; the host caps the number
 // of passes, so the closure always drains.
 #include <algorithm>
@@ -967,20 +969,8 @@ struct Rows {
     {
         double scale = 0.0, ssq = 1.0;
 #pragma unroll 1
-        for (int i = 0; i < NM; ++i) {
-            const double xi = bc_dyn(x, i);
-            const double a = fabs(xi);
-            const bool up = scale < a;
-            const double q = (up ? scale : a) / (up ? a : scale);
-            if (xi != 0.0) {
-                if (up) {
-                    ssq = 1.0 + ssq * (q * q);
-                    scale = a;
-                } else {
-                    ssq = ssq + q * q;
-                }
-            }
-        }
+        for (int i = 0; i < NM; ++i)
+            dnrm2_term(bc_dyn(x, i), scale, ssq);
         return scale * sqrt(ssq);
     }
 
