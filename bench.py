@@ -410,8 +410,9 @@ def main():
              "rung_agreement": round(float((main_r["reg"] == base_r["reg"]).mean()), 6)}
 
     # roofline of the path's matrix-core sweep kernel.  The FP64 path's sweep: the Hessian
-    # H = M^T diag(w e) M on the FP64 matrix cores, 2 nq nm^2 flops per cell-sweep, against the
-    # FP64 matrix peak.  The mixed sweep (mixed_sweep_work): FP64 exponent and gradient
+    # H = M^T diag(w e) M on the FP64 matrix cores, its nm (nm + 1) / 2 distinct entries at 2 nq
+    # flops each, against the FP64 matrix peak; issued: the lower triangle's 4 x 4 blocks that
+    # the kernel forms.  The mixed sweep (mixed_sweep_work): FP64 exponent and gradient
     # products plus the split FP16 pair products of the Hessian, in FP64-equivalent flops
     # against the FP64 matrix peak, i.e. the fraction of the kernel's time its matrix work
     # would take at the published peaks; the rest is its FP64 vector work (exp) and stalls.
@@ -426,13 +427,18 @@ def main():
             kern = (f"{mixed_sweep_kernel(nm)} (mixed phase: FP64 matrix-core exponents and "
                     "gradient, Hessian as split FP16 pair products)")
         else:
-            fl = 2.0 * nq * nm * nm
+            fl = nq * nm * (nm + 1.0)
             kern = f"k_sweep<{nm}> (FP64 MFMA Hessian)"
         ach = fl * cs / secs / 1e12 if ms > 0 else 0.0
         r = {"bound": "mfma", "achieved": round(ach, 3), "peak": FP64_MFMA_PEAK,
              "unit": "TFLOP/s", "frac": round(ach / FP64_MFMA_PEAK, 4), "traffic": None,
              "kernel": kern, "flops_per_cell_sweep": fl, "cell_sweeps_per_step": int(cs),
              "kernel_ms_per_step": round(ms, 3)}
+        if not mixed_kernel:
+            nr = (nm + 3) // 4
+            r["basis"] = "the Hessian's distinct entries, 2 nq flops each"
+            r["matrix_work_issued"] = round(16.0 * nq * nr * (nr + 1) * cs / secs / 1e12, 3) \
+                if ms > 0 else 0.0
         if mixed_kernel:
             r["basis"] = ("FP64-equivalent flops: FP64 matrix work plus FP16 matrix work x "
                           f"{FP64_MFMA_PEAK} / {FP16_MFMA_PEAK}")
