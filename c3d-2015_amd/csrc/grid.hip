@@ -278,7 +278,7 @@ __device__ __forceinline__ double div_by(double x, double d, double r)
 //   - D ordinates' values in flight per thread: 2 where waves enough hide the latency, 4 on
 //     grids that leave the chip mostly idle;
 //   - the ordinate table as scalar operands, issued a stage ahead;
-//   - the tiling above, for the L2.
+//   - the tiling of c3d_tile.h, for the L2.
 // All of it gives the general path's bits as long as the ansatz is zero or within [tiny, kTame]
 // and spacings, theta and the ordinates are within reason (launch_stencil): a value outside of
 // that, or a NaN, anywhere (*wild, from k_ansatz) sends the whole call down the general path.
@@ -290,9 +290,10 @@ __device__ __forceinline__ double div_by(double x, double d, double r)
 // without a division (P2), 1e-270 keeps the slopes' factors of two exact.
 //
 // Measured, ansatz and stencil together, against a kernel with 13 loads, the nested limiter and
-// divisions: M_3 Q = 12 61x45x77 theta = 2: 945 -> 760 us; 96x128x128: 5.80 -> 4.60 ms; 16x12x20:
-// 535 -> 220 us; M_2 20^3 step, flux share: 220 -> 80 us.  The vector unit is busy 56% of the
-// large grid's time (855 M instructions); the L1 serves 10 unaligned rows per cell and ordinate.
+// divisions: M_3 Q = 12 theta = 2 61x45x77: 945 -> 760 us; 96x128x128: 5.64 -> 4.50 ms; 16x12x20:
+// 545 -> 207 us; M_2 Q = 8 20^3 218 -> 79 us, 128^3 3.02 -> 2.53 ms.  At M_2 128^3 (theta 1, powers of
+// two) it issues 97 vector instructions per cell and ordinate, the vector unit busy 46% of the
+// time; the L1 serves 10 unaligned rows per cell and ordinate.
 // The fast path's registers set the waves of a SIMD (D = 2); the general path gets by with them.
 constexpr int stencil_waves(int nm, int d) { return d > 2 ? 1 : (nm == 4 ? 6 : (nm == 9 ? 5 : 4)); }
 template <int NM, bool P2, bool TH1, int D>
