@@ -111,13 +111,14 @@ __device__ __forceinline__ void use_s(const double (&x)[N])
 // uniform and come as scalar operands, half a row ahead; from LDS they took longer than the
 // vector work at M_4.  Small grids share out the ordinates over the blocks.
 // *wild is set where a value is not a number, exceeds kTame, or is not zero but below tiny (see
-// k_stencil), in a cell that some stencil reads.
+// k_stencil), in a cell that some stencil reads; of an exponential the argument is tested instead,
+// |x - ra| <= rb, which is one comparison (M_3 61x45x77: 1% of the flux).
 constexpr double kTame = 1e290;
 template <int NM>
-__global__ __launch_bounds__(kTB) void k_ansatz(Grid G, int64_t ng, int nq, int nqPer,
+__global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(NM == 25 ? 5 : 1))) void k_ansatz(Grid G, int64_t ng, int nq, int nqPer,
                                                  const double *__restrict__ ord,
                                                  const double *__restrict__ alpha, double *A,
-                                                 int isPn, double tiny, int *wild)
+                                                 int isPn, double ra, double rb, int *wild)
 {
     constexpr int HA = (NM + 1) / 2, HB = NM - HA;
     const int64_t cell = (int64_t)blockIdx.x * kTB + threadIdx.x;
@@ -159,7 +160,10 @@ __global__ __launch_bounds__(kTB) void k_ansatz(Grid G, int64_t ng, int nq, int 
         for (int m = 0; m < HB; ++m)
             kin += a[HA + m] * mB[m];
         const double v = isPn == 1 ? kin : (isPn == 2 ? det_exp(kin) : exp(kin));
-        bad |= !(fabs(v) <= kTame) || (fabs(v) < tiny && v != 0.0);
+        if (isPn == 1)
+            bad |= !(fabs(v) <= rb) || (fabs(v) < ra && v != 0.0);
+        else
+            bad |= !(fabs(kin - ra) <= rb);
         if (have)
             *At = v;
         At += ng;
@@ -294,8 +298,9 @@ __device__ __forceinline__ double div_by(double x, double d, double r)
 // 545 -> 207 us; M_2 Q = 8 20^3 218 -> 79 us, 128^3 3.02 -> 2.53 ms.  At M_2 128^3 (theta 1, powers of
 // two) it issues 97 vector instructions per cell and ordinate, the vector unit busy 46% of the
 // time; the L1 serves 10 unaligned rows per cell and ordinate.
-// The fast path's registers set the waves of a SIMD (D = 2); the general path gets by with them.
-constexpr int stencil_waves(int nm, int d) { return d > 2 ? 1 : (nm == 4 ? 6 : (nm == 9 ? 5 : 4)); }
+// The waves of a SIMD that the fast path's registers leave room for (D = 2), for the general path
+// and the Euler stage to keep to.
+constexpr int stencil_waves(int nm, int d) { return d > 2 ? 1 : (nm <= 9 ? 5 : 4); }
 template <int NM, bool P2, bool TH1, int D>
 __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(stencil_waves(NM, D)))) void k_stencil(StencilArgs S, const double *__restrict__ A,
                                                   const double *__restrict__ ord,
@@ -960,6 +965,11 @@ hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *a
     // kind: 1 linear (P_N), 2 deterministic exp (reference-order mode), 0 device exp
     if (!isPn && ctx->precision == C3D_PREC_FP64_REFORDER)
         isPn = 2;
+    // k_ansatz's range: magnitudes, or an exponent's middle and half width (a little less: the
+    // exponentials round)
+    const double lo = log(tiny), hi = log(kTame);
+    const double ra = isPn == 1 ? tiny : 0.5 * (lo + hi);
+    const double rb = isPn == 1 ? kTame : 0.5 * (hi - lo) - 1e-6;
     const Grid G = make_grid(nx, ny, nz);
     const int64_t ng = (int64_t)G.NX * G.NY * G.NZ;
     const int nq = ctx->t.nq;
@@ -972,7 +982,7 @@ hipError_t launch_ansatz(c3d_ctx_s *ctx, int nx, int ny, int nz, const double *a
     hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, ctx->d_wild);
 #define C3D_ANSATZ(NMV)                                                                        \
     hipLaunchKernelGGL(k_ansatz<NMV>, grid, dim3(kTB), 0, s, G, ng, nq, nqPer, ctx->d_ord, \
-                       alpha, A, isPn, tiny, ctx->d_wild)
+                       alpha, A, isPn, ra, rb, ctx->d_wild)
     switch (ctx->t.nm) {
     case 4: C3D_ANSATZ(4); break;
     case 9: C3D_ANSATZ(9); break;
