@@ -604,7 +604,7 @@ constexpr int moment_lds()
 
 // One thread per interior cell.  Bound by the vector unit (six NM x NM products without FMA
 // contraction) and, close behind, by HBM.  A lane that reads its own cell's moments touches a
-// cache line of its own per load (36 lines a load at nm = 9, which bound the kernel), so each
+// cache line of its own per load (36 lines a load at nm = 9), so each
 // wave reads the 64 cells of a stencil offset as one contiguous run, forms the differences on
 // the runs (they are elementwise) and turns only those to a cell per lane through its own LDS
 // rows.  opsT holds the operators' columns: uniform over the wave, they come as scalar
